@@ -121,7 +121,7 @@ def build_oracle() -> None:
 
 
 def build_ref() -> bool:
-    if not os.path.isdir(REFERENCE):
+    if not os.path.exists(os.path.join(REFERENCE, "timestep.c")):
         print("reference sources not mounted: oracle/_ref not rebuilt", flush=True)
         return False
     _run(["make", "-s", "-j4", "-f", os.path.join(REPO, "oracle", "ref", "Makefile"),
