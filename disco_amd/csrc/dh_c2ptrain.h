@@ -14,6 +14,8 @@
 //   KAdam     one thread per trainable parameter (Kingma & Ba 2015, with
 //             bias correction).
 // ReLU's derivative at 0 is taken as 0.
+// The GPU runs the same batch as k_mlp_batch and k_mlp_sum (dh_c2pgrad.h);
+// these functors are its row-by-row form, which the host build runs.
 #pragma once
 #include <math.h>
 
@@ -145,39 +147,14 @@ struct KAdam {
    float *prm, *m, *v;  // prm: the parameter block; m, v: [C2PNET_NTRAIN]
    const float *grad;
    float lr, b1, b2, eps, c1, c2;  // c1 = 1 - b1^step, c2 = 1 - b2^step
-   DHD void operator()(long t) const
+   DHD void operator()(long t) const { step(t, grad[t]); }
+   DHD void step(long t, float g) const
    {
-      float g = grad[t];
       float mt = b1 * m[t] + (1.0f - b1) * g;
       float vt = b2 * v[t] + (1.0f - b2) * g * g;
       m[t] = mt;
       v[t] = vt;
       prm[C2PNET_TRAIN0 + t] -= lr * (mt / c1) / (sqrtf(vt / c2) + eps);
-   }
-};
-
-// The entries of a gradient block outside the trainable range (the
-// normalisation constants), cleared: thread q < C2PNET_TRAIN0 takes entry q,
-// the others the entries after the trainable range.
-struct KGradFrame {
-   float *grad;  // [C2PNET_NPARAM]
-   DHD void operator()(long q) const
-   {
-      grad[q < C2PNET_TRAIN0 ? q : q + C2PNET_NTRAIN] = 0.0f;
-   }
-};
-
-// The mean loss of n rows, L = sum of the rows' squared errors / (2 n), summed
-// in double in row order (one thread).
-struct KLossMean {
-   const float *loss;
-   long n;
-   float *out;
-   DHD void operator()(long) const
-   {
-      double s = 0.0;
-      for (long b = 0; b < n; ++b) s += loss[b];
-      *out = (float)(s / (2.0 * n));
    }
 };
 

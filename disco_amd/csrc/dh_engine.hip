@@ -14,6 +14,7 @@
 
 #include "disco_hip.h"
 #include "dh_pipeline.h"
+#include "dh_c2pgrad.h"
 
 using namespace dh;
 
@@ -755,6 +756,32 @@ struct HipExec {
    int put(void *dst, const void *src, size_t bytes)
    {
       HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
+   // One batch of the learned guess's model (dh_c2pgrad.h): its gradient
+   // and mean loss, or a training step that adds the batch's loss to *total.
+   static size_t mlp_workspace() { return MLP_WS_FLOATS; }
+   static int mlp_launch(const MlpBatch &B, float *ws, float *grad, const MlpAdam &A, float *mean,
+                         float *total, hipStream_t st)
+   {
+      unsigned nwg = mlp_workgroups(B.nb);
+      double *lossp = (double *)ws;
+      float *part = ws + 2 * MLP_MAX_WG;
+      k_mlp_batch<<<nwg, MLP_TPB, 0, st>>>(B.prm, B.X, B.Y, B.idx, B.nb, lossp, part);
+      LAUNCH_CHECK();
+      k_mlp_sum<<<MLP_SUM_BLOCKS + 1, MLP_TPB, 0, st>>>(part, lossp, (int)nwg, B.nb, grad, A, mean,
+                                                        total);
+      LAUNCH_CHECK();
+      return DH_OK;
+   }
+   int mlp_grad(const MlpBatch &B, float *ws, float *grad, float *mean)
+   {
+      return mlp_launch(B, ws, grad, MlpAdam{}, mean, nullptr, stream);
+   }
+   int mlp_train(const MlpBatch &B, float *ws, const KAdam &a, float *total)
+   {
+      return mlp_launch(B, ws, nullptr, MlpAdam{a.prm, a.m, a.v, a.lr, a.b1, a.b2, a.eps, a.c1, a.c2},
+                        nullptr, total, stream);
+   }
+
       HIPCHK(hipStreamSynchronize(stream));
       return DH_OK;
    }
@@ -1218,16 +1245,15 @@ static int ens_launch(dh_ens *e, const EnsLaunch &L)
 
 // ---------------------------------------------------------------------------
 // The learned guess's loss gradient without allocation (dh_c2p_grad_noalloc).
-// The per-row activations and losses of dh_c2p_grad live in `scratch`, one
-// file-scope device array: DH_C2P_NOALLOC_MAX_ROWS rows of C2PNET_ROW
-// activations, then one loss per row.  Host code reaches it through the
-// address hipGetSymbolAddress gives on each device (each GPU holds its own
-// copy), looked up once per device with that device current.  Every row the
-// kernels read is written first in the same call, so nothing needs clearing.
+// The workgroups' partial gradients and losses (dh_c2pgrad.h) live in
+// `scratch`, one file-scope device array of the size any batch needs.  Host
+// code reaches it through the address hipGetSymbolAddress gives on each
+// device (each GPU holds its own copy), looked up once per device with that
+// device current.  Every value k_mlp_sum reads is written first in the same
+// call, so nothing needs clearing.
 // ---------------------------------------------------------------------------
 constexpr long C2P_NOALLOC_ROWS = DH_C2P_NOALLOC_MAX_ROWS;
-constexpr size_t C2P_SCRATCH_FLOATS = (size_t)C2P_NOALLOC_ROWS * (C2PNET_ROW + 1);
-static __device__ __align__(256) float scratch[C2P_SCRATCH_FLOATS];
+static __device__ __align__(256) float scratch[MLP_WS_FLOATS];
 
 constexpr int SCRATCH_MAX_DEVICES = 64;
 static std::mutex g_scratch_mu;
@@ -1465,18 +1491,8 @@ int dh_c2p_grad_noalloc(const float *params, const float *X, const float *Y, lon
    float *s = nullptr;
    DH_TRY(scratch_of_current_device(&s));
    hipStream_t st = (hipStream_t)stream;
-   MlpBatch B{params, X, Y, nullptr, (int)n, s, s + (size_t)n * C2PNET_ROW};
-   k_run<KMlpRow><<<nblocks(n), TPB, 0, st>>>(KMlpRow{B}, n);
-   LAUNCH_CHECK();
-   k_run<KMlpGrad><<<nblocks(C2PNET_NTRAIN), TPB, 0, st>>>(KMlpGrad{B, grad + C2PNET_TRAIN0},
-                                                           C2PNET_NTRAIN);
-   LAUNCH_CHECK();
-   long nframe = C2PNET_NPARAM - C2PNET_NTRAIN;
-   k_run<KGradFrame><<<nblocks(nframe), TPB, 0, st>>>(KGradFrame{grad}, nframe);
-   LAUNCH_CHECK();
-   k_run<KLossMean><<<1, TPB, 0, st>>>(KLossMean{B.loss, n, loss}, 1);
-   LAUNCH_CHECK();
-   return DH_OK;
+   return HipExec::mlp_launch(MlpBatch{params, X, Y, nullptr, (int)n, nullptr, nullptr}, s, grad,
+                              MlpAdam{}, loss, nullptr, (hipStream_t)stream);
 }
 
 int dh_ens_create(dh_ctx *const *members, int n, dh_ens **out)

@@ -1192,6 +1192,17 @@ int c2p_grad(X &x, const float *prm, const float *Xh, const float *Yh, long n, f
 // as lr (1 + cos(pi e / epochs)) / 2; batches of a seeded permutation of
 // the rows each epoch.  Writes the parameter block and the mean loss of the
 // last epoch.
+// Whether an executor runs the model's batches as kernels of its own
+// (mlp_batch) rather than as the functors of dh_c2ptrain.h.
+template <class X, class = void>
+struct HasMlpKernels {
+   static constexpr bool value = false;
+};
+template <class X>
+struct HasMlpKernels<X, decltype((void)&X::mlp_workspace)> {
+   static constexpr bool value = true;
+};
+
 template <class X>
 int c2p_train(X &x, const float *Xh, const float *Yh, long n, int epochs, int batch, float lr,
               unsigned long long seed, float *prm_out, float *loss_out)
@@ -1206,6 +1217,19 @@ int c2p_train(X &x, const float *Xh, const float *Yh, long n, int epochs, int ba
       double bound = 1.0 / sqrt((double)fan_in);
       for (int i = 0; i < count; ++i) prm[w + i] = (float)((2.0 * rng.uniform() - 1.0) * bound);
       for (int i = 0; i < count / fan_in; ++i) prm[b + i] = (float)((2.0 * rng.uniform() - 1.0) * bound);
+   if constexpr (HasMlpKernels<X>::value) {
+      float *ws;
+      DH_TRY(alloc_n(x, &ws, sizeof(float) * x.mlp_workspace()));
+      DH_TRY(alloc_n(x, &g, sizeof(float) * C2PNET_NPARAM));
+      DH_TRY(alloc_n(x, &loss, sizeof(float)));
+      DH_TRY(x.put(dX, Xh, sizeof(float) * C2PNET_IN * n));
+      DH_TRY(x.put(dY, Yh, sizeof(float) * C2PNET_OUT * n));
+      DH_TRY(x.put(dp, prm, sizeof(float) * C2PNET_NPARAM));
+      DH_TRY(x.mlp_grad(MlpBatch{dp, dX, dY, nullptr, (int)n, nullptr, nullptr}, ws, g, loss));
+      DH_TRY(x.get(grad_out, g, sizeof(float) * C2PNET_NPARAM));
+      if (loss_out) DH_TRY(x.get(loss_out, loss, sizeof(float)));
+      return DH_OK;
+   }
    };
    init(C2PNET_W1, C2PNET_B1, C2PNET_IN, C2PNET_IN * C2PNET_H);
    init(C2PNET_W2, C2PNET_B2, C2PNET_H, C2PNET_H * C2PNET_H);
@@ -1217,9 +1241,15 @@ int c2p_train(X &x, const float *Xh, const float *Yh, long n, int epochs, int ba
    DH_TRY(alloc_n(x, &dp, sizeof(float) * C2PNET_NPARAM));
    DH_TRY(alloc_n(x, &m, sizeof(float) * C2PNET_NTRAIN));
    DH_TRY(alloc_n(x, &v, sizeof(float) * C2PNET_NTRAIN));
-   DH_TRY(alloc_n(x, &g, sizeof(float) * C2PNET_NTRAIN));
-   DH_TRY(alloc_n(x, &act, sizeof(float) * C2PNET_ROW * batch));
-   DH_TRY(alloc_n(x, &loss, sizeof(float) * batch));
+   constexpr bool kernels = HasMlpKernels<X>::value;
+   if constexpr (kernels) {
+      DH_TRY(alloc_n(x, &act, sizeof(float) * x.mlp_workspace()));
+      g = loss = nullptr;
+   } else {
+      DH_TRY(alloc_n(x, &g, sizeof(float) * C2PNET_NTRAIN));
+      DH_TRY(alloc_n(x, &act, sizeof(float) * C2PNET_ROW * batch));
+      DH_TRY(alloc_n(x, &loss, sizeof(float) * batch));
+   }
    DH_TRY(alloc_n(x, &eloss, sizeof(float)));
    DH_TRY(alloc_n(x, &idx, sizeof(int) * n));
    DH_TRY(x.put(dX, Xh, sizeof(float) * C2PNET_IN * n));
@@ -1247,11 +1277,15 @@ int c2p_train(X &x, const float *Xh, const float *Yh, long n, int epochs, int ba
          MlpBatch B{dp, dX, dY, idx + s0, nb, act, loss};
          p1 *= b1;
          p2 *= b2;
-         DH_TRY(x.run("c2p_row", KMlpRow{B}, nb));
-         DH_TRY(x.run("c2p_grad", KMlpGrad{B, g}, C2PNET_NTRAIN));
-         DH_TRY(x.run("c2p_adam", KAdam{dp, m, v, g, lre, b1, b2, 1e-8f, (float)(1.0 - p1),
-                                        (float)(1.0 - p2)}, C2PNET_NTRAIN));
-         DH_TRY(x.run("c2p_loss", KLossSum{loss, nb, eloss}, 1));
+         KAdam adam{dp, m, v, g, lre, b1, b2, 1e-8f, (float)(1.0 - p1), (float)(1.0 - p2)};
+         if constexpr (kernels) {
+            DH_TRY(x.mlp_train(B, act, adam, eloss));
+         } else {
+            DH_TRY(x.run("c2p_row", KMlpRow{B}, nb));
+            DH_TRY(x.run("c2p_grad", KMlpGrad{B, g}, C2PNET_NTRAIN));
+            DH_TRY(x.run("c2p_adam", adam, C2PNET_NTRAIN));
+            DH_TRY(x.run("c2p_loss", KLossSum{loss, nb, eloss}, 1));
+         }
       }
       DH_TRY(x.get(&last, eloss, sizeof(float)));
       last = (float)(last / (2.0 * n));

@@ -273,8 +273,8 @@ int dh_c2p_grad(const float *params, const float *X, const float *Y, long n, flo
  * params[4886], X[n][8], Y[n][2], grad[4886] and loss[1] are DEVICE
  * pointers; the kernels are queued on `stream` (a hipStream_t; NULL is the
  * default stream) and the call returns without waiting for them.  n is at
- * most DH_C2P_NOALLOC_MAX_ROWS: the per-row activations live in one fixed
- * device array per GPU (4.2 MB, held until the process ends), shared by
+ * most DH_C2P_NOALLOC_MAX_ROWS: the workgroups' partial sums live in one
+ * fixed device array per GPU (2.5 MB, held until the process ends), shared by
  * every call on that GPU, so calls that overlap on one GPU race.  The
  * results equal dh_c2p_grad's bit for bit. */
 #define DH_C2P_NOALLOC_MAX_ROWS 4096
