@@ -731,31 +731,6 @@ struct HipExec {
       return DH_OK;
    }
 
-   int alloc(void **p, size_t bytes)
-   {
-      if (bytes == 0) bytes = 8;
-      hipError_t e = hipMalloc(p, bytes);
-      if (e != hipSuccess)
-         return fail(DH_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
-      allocs.push_back(*p);
-      return DH_OK;
-   }
-   // Frees one allocation of this executor (after the work queued on it).
-   int release(void *p)
-   {
-      if (!p) return DH_OK;
-      HIPCHK(hipStreamSynchronize(stream));
-      for (size_t i = 0; i < allocs.size(); ++i)
-         if (allocs[i] == p) {
-            allocs.erase(allocs.begin() + (long)i);
-            HIPCHK(hipFree(p));
-            return DH_OK;
-         }
-      return fail(DH_EINVAL, "release of an unknown pointer");
-   }
-   int put(void *dst, const void *src, size_t bytes)
-   {
-      HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
    // One batch of the learned guess's model (dh_c2pgrad.h): its gradient
    // and mean loss, or a training step that adds the batch's loss to *total.
    static size_t mlp_workspace() { return MLP_WS_FLOATS; }
@@ -782,6 +757,31 @@ struct HipExec {
                         nullptr, total, stream);
    }
 
+   int alloc(void **p, size_t bytes)
+   {
+      if (bytes == 0) bytes = 8;
+      hipError_t e = hipMalloc(p, bytes);
+      if (e != hipSuccess)
+         return fail(DH_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+      allocs.push_back(*p);
+      return DH_OK;
+   }
+   // Frees one allocation of this executor (after the work queued on it).
+   int release(void *p)
+   {
+      if (!p) return DH_OK;
+      HIPCHK(hipStreamSynchronize(stream));
+      for (size_t i = 0; i < allocs.size(); ++i)
+         if (allocs[i] == p) {
+            allocs.erase(allocs.begin() + (long)i);
+            HIPCHK(hipFree(p));
+            return DH_OK;
+         }
+      return fail(DH_EINVAL, "release of an unknown pointer");
+   }
+   int put(void *dst, const void *src, size_t bytes)
+   {
+      HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
       HIPCHK(hipStreamSynchronize(stream));
       return DH_OK;
    }

@@ -1145,6 +1145,17 @@ inline void c2p_normalisation(const float *Xh, const float *Yh, long n, float *p
    }
 }
 
+// Whether an executor runs the model's batches as kernels of its own
+// (mlp_batch) rather than as the functors of dh_c2ptrain.h.
+template <class X, class = void>
+struct HasMlpKernels {
+   static constexpr bool value = false;
+};
+template <class X>
+struct HasMlpKernels<X, decltype((void)&X::mlp_workspace)> {
+   static constexpr bool value = true;
+};
+
 // The gradient of the mean loss over all n rows (host arrays) with respect
 // to the parameter block (zero at the normalisation constants), and the
 // loss.
@@ -1159,6 +1170,19 @@ int c2p_grad(X &x, const float *prm, const float *Xh, const float *Yh, long n, f
    DH_TRY(alloc_n(x, &dX, sizeof(float) * C2PNET_IN * n));
    DH_TRY(alloc_n(x, &dY, sizeof(float) * C2PNET_OUT * n));
    DH_TRY(alloc_n(x, &dp, sizeof(float) * C2PNET_NPARAM));
+   if constexpr (HasMlpKernels<X>::value) {
+      float *ws;
+      DH_TRY(alloc_n(x, &ws, sizeof(float) * x.mlp_workspace()));
+      DH_TRY(alloc_n(x, &g, sizeof(float) * C2PNET_NPARAM));
+      DH_TRY(alloc_n(x, &loss, sizeof(float)));
+      DH_TRY(x.put(dX, Xh, sizeof(float) * C2PNET_IN * n));
+      DH_TRY(x.put(dY, Yh, sizeof(float) * C2PNET_OUT * n));
+      DH_TRY(x.put(dp, prm, sizeof(float) * C2PNET_NPARAM));
+      DH_TRY(x.mlp_grad(MlpBatch{dp, dX, dY, nullptr, (int)n, nullptr, nullptr}, ws, g, loss));
+      DH_TRY(x.get(grad_out, g, sizeof(float) * C2PNET_NPARAM));
+      if (loss_out) DH_TRY(x.get(loss_out, loss, sizeof(float)));
+      return DH_OK;
+   }
    DH_TRY(alloc_n(x, &idx, sizeof(int) * n));
    DH_TRY(alloc_n(x, &act, sizeof(float) * C2PNET_ROW * n));
    DH_TRY(alloc_n(x, &loss, sizeof(float) * n));
@@ -1192,17 +1216,6 @@ int c2p_grad(X &x, const float *prm, const float *Xh, const float *Yh, long n, f
 // as lr (1 + cos(pi e / epochs)) / 2; batches of a seeded permutation of
 // the rows each epoch.  Writes the parameter block and the mean loss of the
 // last epoch.
-// Whether an executor runs the model's batches as kernels of its own
-// (mlp_batch) rather than as the functors of dh_c2ptrain.h.
-template <class X, class = void>
-struct HasMlpKernels {
-   static constexpr bool value = false;
-};
-template <class X>
-struct HasMlpKernels<X, decltype((void)&X::mlp_workspace)> {
-   static constexpr bool value = true;
-};
-
 template <class X>
 int c2p_train(X &x, const float *Xh, const float *Yh, long n, int epochs, int batch, float lr,
               unsigned long long seed, float *prm_out, float *loss_out)
@@ -1217,19 +1230,6 @@ int c2p_train(X &x, const float *Xh, const float *Yh, long n, int epochs, int ba
       double bound = 1.0 / sqrt((double)fan_in);
       for (int i = 0; i < count; ++i) prm[w + i] = (float)((2.0 * rng.uniform() - 1.0) * bound);
       for (int i = 0; i < count / fan_in; ++i) prm[b + i] = (float)((2.0 * rng.uniform() - 1.0) * bound);
-   if constexpr (HasMlpKernels<X>::value) {
-      float *ws;
-      DH_TRY(alloc_n(x, &ws, sizeof(float) * x.mlp_workspace()));
-      DH_TRY(alloc_n(x, &g, sizeof(float) * C2PNET_NPARAM));
-      DH_TRY(alloc_n(x, &loss, sizeof(float)));
-      DH_TRY(x.put(dX, Xh, sizeof(float) * C2PNET_IN * n));
-      DH_TRY(x.put(dY, Yh, sizeof(float) * C2PNET_OUT * n));
-      DH_TRY(x.put(dp, prm, sizeof(float) * C2PNET_NPARAM));
-      DH_TRY(x.mlp_grad(MlpBatch{dp, dX, dY, nullptr, (int)n, nullptr, nullptr}, ws, g, loss));
-      DH_TRY(x.get(grad_out, g, sizeof(float) * C2PNET_NPARAM));
-      if (loss_out) DH_TRY(x.get(loss_out, loss, sizeof(float)));
-      return DH_OK;
-   }
    };
    init(C2PNET_W1, C2PNET_B1, C2PNET_IN, C2PNET_IN * C2PNET_H);
    init(C2PNET_W2, C2PNET_B2, C2PNET_H, C2PNET_H * C2PNET_H);
