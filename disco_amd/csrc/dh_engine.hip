@@ -32,19 +32,92 @@ __global__ __launch_bounds__(TPB) void k_run(K k, long n)
    if (t < n) k(t);
 }
 
-// The same with the workgroups renumbered so that each XCD runs one
-// contiguous eighth of the elements (workgroups are dispatched to the XCDs
+// Workgroup b of a launch; with xcd set renumbered so that each XCD runs one
+// contiguous eighth of the workgroups (they are dispatched to the XCDs
 // round-robin, block b to XCD b mod 8): the neighbouring annuli a kernel
 // gathers from then stay in that XCD's L2.  Measured faster only for the
 // kernels that declare xcd_contiguous (the r slopes and the face lists);
 // streaming kernels run slower with it.
-template <class K>
-__global__ __launch_bounds__(TPB) void k_run_xcd(K k, long n)
+__device__ __forceinline__ unsigned block_of(int xcd)
 {
-   unsigned per = gridDim.x / NXCD;
-   unsigned lb = (blockIdx.x % NXCD) * per + blockIdx.x / NXCD;
-   long t = (long)lb * blockDim.x + threadIdx.x;
+   unsigned b = blockIdx.x;
+   return xcd ? (b % NXCD) * (gridDim.x / NXCD) + b / NXCD : b;
+}
+
+// A kernel over cells or faces by elements.
+template <class K>
+__global__ __launch_bounds__(TPB) void k_elems(K k, long n, int xcd)
+{
+   long t = (long)block_of(xcd) * TPB + threadIdx.x;
    if (t < n) k(t);
+}
+
+// A kernel over cells or faces by tiles: one wavefront per tile.  Per lane
+// only the element remains: the annulus or pair, its offsets, ring starts
+// and geometry are uniform and go through the scalar unit, where by
+// elements every kernel begins with two or three dependent vector loads
+// (cjk or pf, then off, Np, I0, fI) and an integer division.  The price is
+// the lanes of each annulus's last tile: by_tiles() has the rule.
+// Measured on the 127 x 31 MHD disk, by elements -> by tiles, us a launch:
+// edge segments 379 -> 309, update 303 -> 286, edges_final 289 -> 266,
+// bfaces_c2p 181 -> 170, update_B 111 -> 102, line steps 91 -> 79; the
+// slopes within 2%; the fluxes, which wait on their arithmetic, 262 -> 264
+// and on annuli of 130 cells (Kerr torus) 285 -> 323.
+// Whether a kernel runs by elements always (its by_elements member).
+template <class K, class = void>
+struct ByElements {
+   static constexpr bool value = false;
+};
+template <class K>
+struct ByElements<K, decltype((void)K::by_elements)> {
+   static constexpr bool value = true;
+};
+template <class K1, class K2>
+struct ByElements<KBoth<K1, K2>> {
+   static constexpr bool value = ByElements<K1>::value || ByElements<K2>::value;
+};
+// Whether the tiles are worth their idle lanes: at least 0.94 of the lanes
+// at work (annuli of 500 cells and more).  At 0.95 (the 127 x 31 disk) a
+// step gains 4%, at 0.92 (the 128-ring vortex) it loses 4%, at 0.8 (the
+// 96 x 48 Kerr torus) 6%.
+static bool by_tiles(const TileList &tl, long n) { return n >= 0.94 * 64.0 * tl.n; }
+
+template <class K>
+__device__ __forceinline__ void tile_wave(const K &k, const TileList &tl, int w, int lane)
+{
+   if (w >= tl.n) return;
+   Tile t = tl.t[w];
+   // (an ensemble's tile comes through a pointer in memory, whose load the
+   // compiler does not know to be uniform)
+   t.first = __builtin_amdgcn_readfirstlane(t.first);
+   t.n = __builtin_amdgcn_readfirstlane(t.n);
+   t.group = __builtin_amdgcn_readfirstlane(t.group);
+   t.dim = __builtin_amdgcn_readfirstlane(t.dim);
+   if (lane < t.n) k.at(t.first + lane, t.group, t.dim);
+}
+template <class K1, class K2>
+__device__ __forceinline__ void tile_wave(const KBoth<K1, K2> &k, const TileList &, int w, int lane)
+{
+   TileList a = k.k1.tiles();
+   if (w < a.n) tile_wave(k.k1, a, w, lane);
+   else tile_wave(k.k2, k.k2.tiles(), w - a.n, lane);
+}
+template <class K>
+DHD TileList tiles_of(const K &k) { return k.tiles(); }
+template <class K1, class K2>
+DHD TileList tiles_of(const KBoth<K1, K2> &k)
+{
+   return {nullptr, tiles_of(k.k1).n + tiles_of(k.k2).n};
+}
+constexpr int WAVES = TPB / 64;
+__device__ __forceinline__ int wave_of(unsigned blk)
+{
+   return __builtin_amdgcn_readfirstlane((int)(blk * WAVES + threadIdx.x / 64));
+}
+template <class K>
+__global__ __launch_bounds__(TPB) void k_tiles(K k, TileList tl, int xcd)
+{
+   tile_wave(k, tl, wave_of(block_of(xcd)), threadIdx.x & 63);
 }
 
 template <class K, class = void>
@@ -77,7 +150,7 @@ struct KZeroWords {
 // annulus scans 64 cells at a time with ballots for the first cell in the
 // first quadrant that follows a cell in the fourth.
 // Block b of the launch (its TPB / 64 wavefronts take annuli 4 b .. 4 b + 3).
-__device__ void ring_start_block(const Mesh &m, const double *piph, int *I0, unsigned blk)
+__device__ __forceinline__ void ring_start_block(const Mesh &m, const double *piph, int *I0, unsigned blk)
 {
    int a = blk * (TPB / 64) + threadIdx.x / 64;
    int lane = threadIdx.x & 63;
@@ -119,7 +192,7 @@ __global__ __launch_bounds__(TPB) void k_ring_start(Mesh m, const double *piph, 
 
 // flip_fluxes (bfields.c:742-814): one wavefront per face track; the lanes
 // read 64 flags at a time and lane 0 hands the flagged faces over in order.
-__device__ void flips_block(const Mesh &m, int dim, const Faces &F, const signed char *flag,
+__device__ __forceinline__ void flips_block(const Mesh &m, int dim, const Faces &F, const signed char *flag,
                             double *Phi, double *rkPhi, unsigned blk)
 {
    int JK = blk * (TPB / 64) + threadIdx.x / 64;
@@ -151,7 +224,7 @@ __global__ __launch_bounds__(TPB) void k_flips(Mesh m, int dim, Faces F, const s
 // then checks each guess against one step of the walk from the guess before
 // it.  A ring with any miss is walked again sequentially, so start[] is the
 // sequential walk's in every case.
-__device__ void bc_scan_block(const Mesh &m, int side, const double *piph, const double *dphi,
+__device__ __forceinline__ void bc_scan_block(const Mesh &m, int side, const double *piph, const double *dphi,
                               int *start, unsigned blk)
 {
    __shared__ int s_first, s_miss;
@@ -215,7 +288,7 @@ __global__ __launch_bounds__(TPB) void k_bc_scan(Mesh m, int side, const double 
 // adds its lanes' sums and thread 0 the waves'.  (The host build sums the
 // cells in order, as the reference does; the two differ by rounding only.)
 template <int KIND>
-__device__ void diag_block(const Mesh &m, const dh_params &P, const DiagPlanet &p1,
+__device__ __forceinline__ void diag_block(const Mesh &m, const dh_params &P, const DiagPlanet &p1,
                            const double *prim, const double *piph, const double *dphi, double dt,
                            double *Qrz, unsigned blk)
 {
@@ -309,7 +382,7 @@ __global__ __launch_bounds__(TPB) void k_report(Mesh m, dh_params P, DiagPlanet 
 constexpr unsigned MINDT_BLOCKS = 2048;
 // Block blk of nb blocks that share the cells (a grid-stride loop).
 template <int NQ, class H>
-__device__ void mindt_block(const Mesh &m, const dh_params &P, const double *prim,
+__device__ __forceinline__ void mindt_block(const Mesh &m, const dh_params &P, const double *prim,
                             const double *piph, const double *dphi, const double *wiph,
                             unsigned long long *out, unsigned blk, unsigned nb)
 {
@@ -484,7 +557,7 @@ struct TimerRow {
 // Launch variants of a kernel that runs over cells or faces (run_tuned):
 // 0 storage order with the workgroups dealt to the XCDs round-robin (the
 // hardware's order), 1 storage order with each XCD given a contiguous
-// eighth (k_run_xcd), 2 + s the group order s of the kernel's OrderSet
+// eighth (block_of), and for a kernel that runs by tiles 2 + s the group order s of the kernel's OrderSet
 // (strips of annuli, XCD-contiguous).  All give the same results.
 struct TuneRow {
    std::string name;
@@ -552,10 +625,7 @@ struct HipExec {
       if (n <= 0) return DH_OK;
       {
          Bracket b(*this, name);
-         if constexpr (XcdContiguous<K>::value)
-            k_run_xcd<K><<<nblocks_xcd(n), TPB, 0, stream>>>(k, n);
-         else
-            k_run<K><<<nblocks(n), TPB, 0, stream>>>(k, n);
+         k_run<K><<<nblocks(n), TPB, 0, stream>>>(k, n);
       }
       LAUNCH_CHECK();
       return DH_OK;
@@ -580,7 +650,9 @@ struct HipExec {
                  const int *strips)
    {
       if (n <= 0) return DH_OK;
-      int row = (int)(&tune_row(name, 2 + nord, strips, XcdContiguous<K>::value ? 1 : 0) -
+      bool tiled = false;
+      if constexpr (!ByElements<K>::value) tiled = by_tiles(tiles_of(k), n);
+      int row = (int)(&tune_row(name, 2 + (tiled ? nord : 0), strips, XcdContiguous<K>::value ? 1 : 0) -
                       tunes.data());
       TuneRow &t = tunes[row];
       int v = t.chosen >= 0 ? t.chosen : t.dflt;
@@ -594,12 +666,13 @@ struct HipExec {
       }
       {
          Bracket b(*this, name);
-         if (v == 0)
-            k_run<K><<<nblocks(n), TPB, 0, stream>>>(k, n);
-         else if (v == 1)
-            k_run_xcd<K><<<nblocks_xcd(n), TPB, 0, stream>>>(k, n);
-         else
-            k_run_xcd<Grouped<K>><<<nblocks_xcd(n), TPB, 0, stream>>>(Grouped<K>{k, ords[v - 2]}, n);
+         if constexpr (!ByElements<K>::value)
+            if (tiled) {
+               TileList tl = v < 2 ? tiles_of(k) : ords[v - 2].tiles;
+               long nt = (long)tl.n * 64;
+               k_tiles<K><<<v == 0 ? nblocks(nt) : nblocks_xcd(nt), TPB, 0, stream>>>(k, tl, v != 0);
+            }
+         if (!tiled) k_elems<K><<<v == 0 ? nblocks(n) : nblocks_xcd(n), TPB, 0, stream>>>(k, n, v);
       }
       LAUNCH_CHECK();
       if (timing) {
@@ -931,10 +1004,20 @@ struct RunOp {
    K k;
    long n;
    unsigned blocks() const { return nblocks(n); }
-   __device__ void run(unsigned b) const
+   __device__ __forceinline__ void run(unsigned b) const
    {
       long t = (long)b * TPB + threadIdx.x;
       if (t < n) k(t);
+   }
+};
+// A kernel over cells or faces by tiles.
+template <class K>
+struct TileOp {
+   K k;
+   unsigned blocks() const { return nblocks((long)tiles_of(k).n * 64); }
+   __device__ __forceinline__ void run(unsigned b) const
+   {
+      tile_wave(k, tiles_of(k), wave_of(b), threadIdx.x & 63);
    }
 };
 struct RingStartOp {
@@ -942,7 +1025,7 @@ struct RingStartOp {
    const double *piph;
    int *I0;
    unsigned blocks() const { return (unsigned)((m.nann + 3) / 4); }
-   __device__ void run(unsigned b) const { ring_start_block(m, piph, I0, b); }
+   __device__ __forceinline__ void run(unsigned b) const { ring_start_block(m, piph, I0, b); }
 };
 struct FlipsOp {
    Mesh m;
@@ -951,7 +1034,7 @@ struct FlipsOp {
    const signed char *flag;
    double *Phi, *rkPhi;
    unsigned blocks() const { return (unsigned)((F.npairs + 3) / 4); }
-   __device__ void run(unsigned b) const { flips_block(m, dim, F, flag, Phi, rkPhi, b); }
+   __device__ __forceinline__ void run(unsigned b) const { flips_block(m, dim, F, flag, Phi, rkPhi, b); }
 };
 struct BcScanOp {
    Mesh m;
@@ -959,7 +1042,7 @@ struct BcScanOp {
    const double *piph, *dphi;
    int *start;
    unsigned blocks() const { return (unsigned)((long)bc_lines(m, side) * bc_layers(m, side)); }
-   __device__ void run(unsigned b) const { bc_scan_block(m, side, piph, dphi, start, b); }
+   __device__ __forceinline__ void run(unsigned b) const { bc_scan_block(m, side, piph, dphi, start, b); }
 };
 template <int NQ, class H>
 struct MindtOp {
@@ -969,7 +1052,7 @@ struct MindtOp {
    unsigned long long *out;
    unsigned nb;
    unsigned blocks() const { return nb; }
-   __device__ void run(unsigned b) const
+   __device__ __forceinline__ void run(unsigned b) const
    {
       mindt_block<NQ, H>(m, P, prim, piph, dphi, wiph, out, b, nb);
    }
@@ -987,24 +1070,21 @@ struct DiagOp {
    const double *prim, *piph, *dphi;
    double *Qrz;
    unsigned blocks() const { return (unsigned)m.nann; }
-   __device__ void run(unsigned b) const
+   __device__ __forceinline__ void run(unsigned b) const
    {
       diag_block<KIND>(m, P, a->p1, prim, piph, dphi, a->dt, Qrz, b);
    }
 };
 
-// Block b of the concatenated table goes to mesh m with boff[m] <= b < boff[m + 1].
+// Block b of the launch is block map[b].y of mesh map[b].x.  One scalar load
+// finds it; a bisection of the meshes' block offsets was a chain of four to
+// six dependent loads at the head of every workgroup.
 template <class Op>
-__global__ __launch_bounds__(TPB) void k_group(const Op *ops, const unsigned *boff, int nm)
+__global__ __launch_bounds__(TPB) void k_group(const Op *__restrict__ ops,
+                                               const int2 *__restrict__ map)
 {
-   unsigned b = blockIdx.x;
-   int lo = 0, hi = nm;
-   while (hi - lo > 1) {
-      int mid = (lo + hi) >> 1;
-      if (boff[mid] <= b) lo = mid;
-      else hi = mid;
-   }
-   ops[lo].run(b - boff[lo]);
+   int2 e = map[blockIdx.x];
+   ops[e.x].run((unsigned)e.y);
 }
 
 // Every mesh's {dt, planets} of the step, one thread per mesh.
@@ -1025,7 +1105,7 @@ struct GroupOp {
    size_t size;
    std::vector<unsigned char> bytes;
    unsigned blocks;
-   void (*launch)(const void *ops, const unsigned *boff, int nm, unsigned total, hipStream_t s);
+   void (*launch)(const void *ops, const int2 *map, unsigned total, hipStream_t s);
 };
 template <class Op>
 struct OpType {
@@ -1034,9 +1114,9 @@ struct OpType {
       static const char t = 0;
       return &t;
    }
-   static void launch(const void *ops, const unsigned *boff, int nm, unsigned total, hipStream_t s)
+   static void launch(const void *ops, const int2 *map, unsigned total, hipStream_t s)
    {
-      if (total) k_group<Op><<<total, TPB, 0, s>>>((const Op *)ops, boff, nm);
+      if (total) k_group<Op><<<total, TPB, 0, s>>>((const Op *)ops, map);
    }
 };
 
@@ -1065,9 +1145,11 @@ struct GroupExec {
       return n > 0 ? rec(RunOp<K>{k, n}) : DH_OK;
    }
    template <class K>
-   int run_tuned(const char *name, const K &k, long n, const GroupOrder *, int, const int *)
+   int run_tuned(const char *, const K &k, long n, const GroupOrder *, int, const int *)
    {
-      return run(name, k, n);
+      if (n <= 0) return DH_OK;
+      if constexpr (ByElements<K>::value) return rec(RunOp<K>{k, n});
+      else return rec(TileOp<K>{k});
    }
    int ring_start(const Mesh &m, const double *piph, int *I0)
    {
@@ -1118,14 +1200,14 @@ struct GroupExec {
 };
 
 // One launch of an ensemble: the ops of every mesh in device memory and
-// their concatenated block table.
+// their block table.
 struct EnsLaunch {
    const void *tag = nullptr;
-   void (*launch)(const void *, const unsigned *, int, unsigned, hipStream_t) = nullptr;
+   void (*launch)(const void *, const int2 *, unsigned, hipStream_t) = nullptr;
    std::vector<unsigned char> host;  // every mesh's op bytes, in mesh order
    unsigned total = 0;
    void *d_ops = nullptr;
-   unsigned *d_boff = nullptr;
+   int2 *d_map = nullptr;
 };
 
 template <int NQ, class H>
@@ -1168,7 +1250,7 @@ struct dh_ens {
 static void ens_free_launch(EnsLaunch &L)
 {
    if (L.d_ops) (void)hipFree(L.d_ops);
-   if (L.d_boff) (void)hipFree(L.d_boff);
+   if (L.d_map) (void)hipFree(L.d_map);
    L = EnsLaunch();
 }
 
@@ -1202,23 +1284,27 @@ static int ens_build_launch(const std::vector<GroupExec> &rec, size_t i, EnsLaun
    int nm = (int)rec.size();
    const GroupOp &g0 = rec[0].ops[i];
    std::vector<unsigned char> host;
-   std::vector<unsigned> boff(nm + 1, 0);
+   unsigned total = 0;
    for (int m = 0; m < nm; ++m) {
       const GroupOp &g = rec[m].ops[i];
       host.insert(host.end(), g.bytes.begin(), g.bytes.end());
-      boff[m + 1] = boff[m] + g.blocks;
+      total += g.blocks;
    }
-   *changed = !(L.d_ops && L.tag == g0.tag && L.host == host && L.total == boff[nm]);
+   *changed = !(L.d_ops && L.tag == g0.tag && L.host == host && L.total == total);
    if (!*changed) return DH_OK;
+   std::vector<int2> map;
+   map.reserve(total);
+   for (int m = 0; m < nm; ++m)
+      for (unsigned b = 0; b < rec[m].ops[i].blocks; ++b) map.push_back(make_int2(m, (int)b));
    ens_free_launch(L);
    L.tag = g0.tag;
    L.launch = g0.launch;
    L.host = std::move(host);
-   L.total = boff[nm];
+   L.total = total;
    HIPCHK(hipMalloc(&L.d_ops, L.host.size()));
-   HIPCHK(hipMalloc((void **)&L.d_boff, sizeof(unsigned) * (nm + 1)));
+   HIPCHK(hipMalloc((void **)&L.d_map, sizeof(int2) * (total ? total : 1)));
    HIPCHK(hipMemcpy(L.d_ops, L.host.data(), L.host.size(), hipMemcpyHostToDevice));
-   HIPCHK(hipMemcpy(L.d_boff, boff.data(), sizeof(unsigned) * (nm + 1), hipMemcpyHostToDevice));
+   if (total) HIPCHK(hipMemcpy(L.d_map, map.data(), sizeof(int2) * total, hipMemcpyHostToDevice));
    return DH_OK;
 }
 
@@ -1238,7 +1324,7 @@ static int ens_check_records(const std::vector<GroupExec> &rec)
 
 static int ens_launch(dh_ens *e, const EnsLaunch &L)
 {
-   L.launch(L.d_ops, L.d_boff, e->nm, L.total, e->stream);
+   L.launch(L.d_ops, L.d_map, L.total, e->stream);
    LAUNCH_CHECK();
    return DH_OK;
 }

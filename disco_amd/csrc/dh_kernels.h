@@ -81,6 +81,7 @@ constexpr int ORDER_CHUNK = 256;
 struct GroupOrder {
    const int *first, *pos, *chunk;
    int ng;
+   TileList tiles;  // the same sequence in tiles (what a wavefront-per-tile launch takes)
    DHD long elem(long t) const
    {
       int p = chunk[t / ORDER_CHUNK];
@@ -89,8 +90,12 @@ struct GroupOrder {
    }
 };
 
-// A kernel run in a group order (its workgroups go to the XCDs in
-// contiguous runs, so that neighbouring groups of the order share an L2).
+// Kernels over cells or faces take an element and its group (and, for both
+// face lists as one range, its direction): at(e, g, dim).  A launch by tiles
+// (one wavefront per tile of tiles()) hands them the tile's group; the
+// element alone, operator()(e), looks its group up.
+
+// A kernel run in a group order, element by element.
 template <class K>
 struct Grouped {
    K k;
@@ -115,6 +120,7 @@ struct KBoth {
 // One direction's face list: faces of annulus pair P are fI[P] .. fI[P+1]-1.
 struct Faces {
    int n, npairs;
+   TileList tiles;  // the faces in storage order
    const int *fI;   // [npairs+1] first face of every annulus pair
    const int *pf;   // [n] annulus pair of every face (static, like fI)
    int *L, *R;
@@ -232,9 +238,10 @@ struct KWcell {
    dh_params P;
    const double *prim;
    double *wiph;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
-      int a = m.cjk[c];
       double w = 0.0;
       if (P.mesh_motion == 4) {
          int j = a % m.Nr;
@@ -276,10 +283,9 @@ struct KWcellAvg {
 // The limited phi slopes of cell c from its two phi neighbours.
 template <int NQ>
 DHD void plm_phi_cell(const Mesh &m, double PLM, const double *prim, const double *dphi, long c,
-                      double *g)
+                      int a, double *g)
 {
    size_t nt = (size_t)m.ntot;
-   int a = m.cjk[c];
    int c0 = m.off[a], np = m.Np[a];
    int i = (int)(c - c0);
    long cL = i == 0 ? c0 + np - 1 : c - 1;
@@ -306,11 +312,13 @@ struct KPlmPhi {
    double PLM;
    const double *prim, *dphi;
    double *gradp;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
       double g[NQ];
-      plm_phi_cell<NQ>(m, PLM, prim, dphi, c, g);
+      plm_phi_cell<NQ>(m, PLM, prim, dphi, c, a, g);
 #pragma unroll
       for (int q = 0; q < NQ; ++q) gradp[q * nt + c] = g[q];
    }
@@ -405,9 +413,10 @@ struct KFaces {
       F.phic[f] = g.phic;
       F.dphi[f] = g.dp;
    }
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
-      int a = m.cjk[c];
       int j = a % m.Nr, k = a / m.Nr;
       if (dim == 1 ? j >= m.Nr - 1 : k >= m.Nz - 1) return;
       CellRanges cr = load_ranges(m, dim, rng, F.fI, c, a);
@@ -439,10 +448,11 @@ struct KCellRanges {
    static constexpr int dim = DIM;
    const double *piph;
    int *rng;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
-      int a = m.cjk[c];
       int i = (int)(c - m.off[a]);
       int j = a % m.Nr, k = a / m.Nr;
       Ring self = make_ring(piph, m, m.I0, a);
@@ -535,10 +545,11 @@ struct KGrad {
          if (S < 0.0) A.neg |= 1u << q;
       }
    }
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
-      int a = m.cjk[c];
       int j = a % m.Nr, k = a / m.Nr;
       CellRanges cr = load_ranges(m, dim, rng, F.fI, c, a);
       double dxLi = 0, dxRi = 0, dxLo = 0, dxRo = 0;
@@ -640,14 +651,16 @@ DHD void add_visc(const dh_params &P, const double *pL, const double *pR, const 
 template <int NQ, class H>
 struct KFluxPhi {
    Mesh m;
+   static constexpr bool by_elements = true;  // bound by its arithmetic: no lane to spare
    dh_params P;
    const double *dtp;
    const double *prim, *gradp, *gradr, *gradz, *piph, *dphi, *wiph;
    double *dFp, *emf_phi;
    DHD bool in_range(int j, int k) const { return phi_in_range(m, IsMHD<H>::value && P.ct, j, k); }
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
-      int a = m.cjk[c];
       int j = a % m.Nr, k = a / m.Nr;
       if (!in_range(j, k)) return;
       size_t nt = (size_t)m.ntot;
@@ -713,16 +726,18 @@ struct KFluxPhi {
 template <int NQ, class H, int DIM>
 struct KFluxTrans {
    Mesh m;
+   static constexpr bool by_elements = true;
    dh_params P;
    static constexpr int dim = DIM;
    const double *dtp;
    Faces F;
    const double *prim, *gradp, *gradr, *gradz, *piph, *dphi;
    double *dF, *emf_face;
-   DHD void operator()(long f) const
+   DHD TileList tiles() const { return F.tiles; }
+   DHD void operator()(long f) const { at(f, F.pf[f], dim); }
+   DHD void at(long f, int Pi, int) const
    {
       constexpr bool mhd = IsMHD<H>::value;
-      int Pi = F.pf[f];
       Pair pr = pair_of(m, dim, Pi);
       if (!pair_has_flux(m, mhd && P.ct, dim, pr.j, pr.k)) return;
       size_t nt = (size_t)m.ntot, nfs = (size_t)F.n;
@@ -967,11 +982,12 @@ struct KUpdate {
    const double *dFp, *dFr, *dFz;
    const int *fIr, *fIz, *rngr, *rngz;
    int nfr, nfz;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       constexpr bool mhd = IsMHD<H>::value;
       size_t nt = (size_t)m.ntot;
-      int a = m.cjk[c];
       int c0 = m.off[a], np = m.Np[a];
       int i = (int)(c - c0);
       int j = a % m.Nr, k = a / m.Nr;
@@ -1082,10 +1098,11 @@ struct KEdgesCollect {
    const int *rngr, *rngz;
    const double *emf_r, *emf_z, *Ecarry;
    double *Epre;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
-      int a = m.cjk[c];
       int c0 = m.off[a], np = m.Np[a];
       long cm = c == c0 ? c0 + np - 1 : c - 1;
       int j = a % m.Nr, k = a / m.Nr;
@@ -1153,12 +1170,11 @@ struct KEdgesCollect {
 
 // avg_Efields, first part (bfields.c:400-441), evaluated where it is read:
 // each phi-edge takes the mean of the values its two cells hold.  Slot s of
-// E (h = 0) or B (h = 1) of cell c.
-DHD double edge_avg(const Mesh &m, const double *Epre, int h, int s, long c)
+// E (h = 0) or B (h = 1) of cell c of annulus a.
+DHD double edge_avg(const Mesh &m, const double *Epre, int h, int s, long c, int a)
 {
    size_t nt = (size_t)m.ntot;
    const double *X = Epre + (size_t)h * 8 * nt;
-   int a = m.cjk[c];
    int c0 = m.off[a], np = m.Np[a];
    int e = s & 3, base = s & 4;
    if (e < 2) {
@@ -1173,23 +1189,23 @@ DHD double edge_avg(const Mesh &m, const double *Epre, int h, int s, long c)
 // face f (of direction dim) is the mean of its owner's value and the other
 // cell's two corner values interpolated in phi; E in *fE, B in *fB.  Each
 // face's edge is read by one cell, the face's owner (edges_post_face), which
-// forms it where it reads it.
-DHD void face_emf(const Mesh &m, int dim, const Faces &F, const double *piph,
+// forms it where it reads it.  The face's cells are of annuli aL and aR.
+DHD void face_emf(const Mesh &m, int dim, int aL, int aR, const Faces &F, const double *piph,
                   const double *dphi, const double *Epre, int f, double *fE, double *fB)
 {
    int L = F.L[f], R = F.R[f];
    int LR = F.LR[f];
    int c1 = LR == 0 ? L : R, c2 = LR == 0 ? R : L;
+   int a1 = LR == 0 ? aL : aR, a2 = LR == 0 ? aR : aL;
    double dp1 = get_dp(piph[c2], piph[c1], m.Pmax);
    double dp2 = dphi[c2] - dp1;
    int eL = dim == 1 ? 1 : 5, eR = dim == 1 ? 0 : 4;
    // LRtype 0: the face ends at L's upper edge; R's corners are interpolated
    int eo = LR == 0 ? eL : eR, ec = LR == 0 ? eR : eL;
-   int co = LR == 0 ? L : R;
-   double Ea = (dp2 * edge_avg(m, Epre, 0, ec, c2) + dp1 * edge_avg(m, Epre, 0, ec + 2, c2)) / (dp1 + dp2);
-   double Ba = (dp2 * edge_avg(m, Epre, 1, ec, c2) + dp1 * edge_avg(m, Epre, 1, ec + 2, c2)) / (dp1 + dp2);
-   *fE = .5 * (edge_avg(m, Epre, 0, eo, co) + Ea);
-   *fB = .5 * (edge_avg(m, Epre, 1, eo, co) + Ba);
+   double Ea = (dp2 * edge_avg(m, Epre, 0, ec, c2, a2) + dp1 * edge_avg(m, Epre, 0, ec + 2, c2, a2)) / (dp1 + dp2);
+   double Ba = (dp2 * edge_avg(m, Epre, 1, ec, c2, a2) + dp1 * edge_avg(m, Epre, 1, ec + 2, c2, a2)) / (dp1 + dp2);
+   *fE = .5 * (edge_avg(m, Epre, 0, eo, c1, a1) + Ea);
+   *fB = .5 * (edge_avg(m, Epre, 1, eo, c1, a1) + Ba);
 }
 
 // The four phi+ edges of a cell after avg_Efields, before the advective
@@ -1202,26 +1218,28 @@ struct EdgeArgs {
    const double *Epre, *piph, *dphi;
 };
 
-DHD void edges_post_face(const EdgeArgs &g, long c, double *out)
+DHD void edges_post_face(const EdgeArgs &g, long c, int a, double *out)
 {
    const Mesh &m = g.m;
-   size_t nt = (size_t)m.ntot;
-   int a = m.cjk[c];
    const int slots[4] = {0, 1, 4, 5};
 #pragma unroll
    for (int s = 0; s < 4; ++s) {
-      out[s] = edge_avg(m, g.Epre, 0, slots[s], c);
-      out[4 + s] = edge_avg(m, g.Epre, 1, slots[s], c);
+      out[s] = edge_avg(m, g.Epre, 0, slots[s], c, a);
+      out[4 + s] = edge_avg(m, g.Epre, 1, slots[s], c, a);
    }
    if (m.Nr > 1) {
       CellRanges cr = load_ranges(m, 1, g.rngr, g.Fr.fI, c, a);
-      if (cr.in) face_emf(m, 1, g.Fr, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[0], &out[4]);
-      if (cr.out) face_emf(m, 1, g.Fr, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[1], &out[5]);
+      if (cr.in)
+         face_emf(m, 1, a - 1, a, g.Fr, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[0], &out[4]);
+      if (cr.out)
+         face_emf(m, 1, a, a + 1, g.Fr, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[1], &out[5]);
    }
    if (m.Nz > 1) {
       CellRanges cr = load_ranges(m, 2, g.rngz, g.Fz.fI, c, a);
-      if (cr.in) face_emf(m, 2, g.Fz, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[2], &out[6]);
-      if (cr.out) face_emf(m, 2, g.Fz, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[3], &out[7]);
+      if (cr.in)
+         face_emf(m, 2, a - m.Nr, a, g.Fz, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[2], &out[6]);
+      if (cr.out)
+         face_emf(m, 2, a, a + m.Nr, g.Fz, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[3], &out[7]);
    }
 }
 
@@ -1234,14 +1252,15 @@ struct KEdgesFinal {
    int ct;
    const double *wiph, *emf_r, *emf_z;
    double *Eo, *Eown, *Ecarry;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return g.m.tiles; }
+   DHD void operator()(long c) const { at(c, g.m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       const Mesh &m = g.m;
       size_t nt = (size_t)m.ntot;
-      int a = m.cjk[c];
       int j = a % m.Nr, k = a / m.Nr;
       double v[8];
-      edges_post_face(g, c, v);
+      edges_post_face(g, c, a, v);
       double own[4] = {0.0, 0.0, 0.0, 0.0};
       if (m.Nr > 1) {
          size_t nfs = (size_t)g.Fr.n;
@@ -1275,7 +1294,7 @@ struct KEdgesFinal {
          int c0 = m.off[a], np = m.Np[a];
          long cm = c == c0 ? c0 + np - 1 : c - 1;
          double vm[8];
-         edges_post_face(g, cm, vm);
+         edges_post_face(g, cm, a, vm);
          double Ec[8] = {E0, E1, vm[0], vm[1], E4, E5, vm[2], vm[3]};
          double Bc[8] = {v[4], v[5], vm[4], vm[5], v[6], v[7], vm[6], vm[7]};
 #pragma unroll
@@ -1309,11 +1328,12 @@ struct KUpdateB {
    const double *Phi;
    const double *rkPhi;
    double *Phi_out;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
       const double dt = *dtp;
-      int a = m.cjk[c];
       int j = a % m.Nr, k = a / m.Nr;
       double ph[5];
 #pragma unroll
@@ -1412,10 +1432,11 @@ struct KLineSteps {
    Mesh m;
    Faces F;
    int *estep;  // [2][F.n]
-   DHD void operator()(long t) const
+   DHD TileList tiles() const { return F.tiles; }
+   DHD void operator()(long t) const { at(t, F.pf[t], DIM); }
+   DHD void at(long t, int JK, int) const
    {
       int f = (int)t;
-      int JK = F.pf[f];
       Pair pr = pair_of(m, DIM, JK);
       int base = F.fI[JK];
       FaceRing self = make_face_ring(F.up, base, F.fI[JK + 1] - base);
@@ -1444,15 +1465,19 @@ struct KEdgeSegments {
    const int *estep_r, *estep_z, *lbase_r, *lbase_z;
    const double *piph, *dphi, *Eown;
    double *seg_r, *seg_z;
+   DHD TileList tiles() const { return m.etiles; }
    DHD void operator()(long t) const
+   {
+      if (t < Fr.n) at(t, Fr.pf[t], 1);
+      else at(t, Fz.pf[t - Fr.n], 2);
+   }
+   DHD void at(long t, int JK, int dim) const
    {
       size_t nt = (size_t)m.ntot;
       const double dt = *dtp;
-      int dim = t < Fr.n ? 1 : 2;
       const Faces &F = dim == 1 ? Fr : Fz;
       const int *estep = dim == 1 ? estep_r : estep_z;
       int f = (int)(dim == 1 ? t : t - Fr.n);
-      int JK = F.pf[f];
       Pair pr = pair_of(m, dim, JK);
       EdgeRole er = edge_role(m, dim, pr.j, pr.k, 1);  // the role where F's list is first
       if (!er.ok) return;
@@ -1501,16 +1526,20 @@ struct KEdgeAdjust {
    const int *estep_r, *estep_z, *lbase_r, *lbase_z;
    const double *seg_r, *seg_z;
    double *Phi;
+   DHD TileList tiles() const { return m.etiles; }
    DHD void operator()(long t) const
    {
+      if (t < Fr.n) at(t, Fr.pf[t], 1);
+      else at(t, Fz.pf[t - Fr.n], 2);
+   }
+   DHD void at(long t, int JK, int dim) const
+   {
       size_t nt = (size_t)m.ntot;
-      int dim = t < Fr.n ? 1 : 2;
       const Faces &F = dim == 1 ? Fr : Fz;
       const int *estep = dim == 1 ? estep_r : estep_z;
       const int *lbase = dim == 1 ? lbase_r : lbase_z;
       const double *segd = dim == 1 ? seg_r : seg_z;
       int f = (int)(dim == 1 ? t : t - Fr.n);
-      int JK = F.pf[f];
       Pair pr = pair_of(m, dim, JK);
       int base = F.fI[JK];
       int N = F.fI[JK + 1] - base;
@@ -1553,9 +1582,10 @@ struct KFlipFlags {
       int o = F.LR[f] == 0 ? F.L[f] : F.R[f];
       return piph[o] + wiph[o] * *dtp;
    }
-   DHD void operator()(long f) const
+   DHD TileList tiles() const { return F.tiles; }
+   DHD void operator()(long f) const { at(f, F.pf[f], DIM); }
+   DHD void at(long f, int JK, int) const
    {
-      int JK = F.pf[f];
       int base = F.fI[JK], N = F.fI[JK + 1] - base;
       int n = (int)f - base;
       int fm = base + (n == 0 ? N - 1 : n - 1);
@@ -1617,10 +1647,11 @@ struct KBfacesC2p {
    int type;    // 0: primitive B (set_B_fields), 1: conserved B
    int do_c2p;  // cons2prim of real cells afterwards
    unsigned char *info;  // GRMHD: each cons2prim's record (C2P_INFO_*), or null
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
-      int a = m.cjk[c];
       int c0 = m.off[a], np = m.Np[a];
       long cm = c == c0 ? c0 + np - 1 : c - 1;
       int j = a % m.Nr, k = a / m.Nr;
@@ -1694,10 +1725,11 @@ struct KC2p {
    double *prim;
    const float *guess;
    unsigned char *info;
-   DHD void operator()(long c) const
+   DHD TileList tiles() const { return m.tiles; }
+   DHD void operator()(long c) const { at(c, m.cjk[c], 0); }
+   DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
-      int a = m.cjk[c];
       int j = a % m.Nr, k = a / m.Nr;
       if (!is_real(m, j, k)) return;
       double rp = m.r_jph[j], rm = m.r_jph[j - 1];

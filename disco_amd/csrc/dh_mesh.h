@@ -15,6 +15,22 @@
 
 namespace dh {
 
+// A run of at most TILE consecutive elements (cells of one annulus, faces of
+// one annulus pair): what one wavefront takes.  The group, and with it
+// every index and geometric factor of the annulus or pair, is the same for
+// all its lanes, so they live in scalar registers and are read by scalar
+// loads.
+constexpr int TILE = 64;
+struct Tile {
+   int first, n;   // first element, count
+   int group;      // annulus or annulus pair
+   int dim;        // faces: 1 (r) or 2 (z); cells: 0
+};
+struct TileList {
+   const Tile *t;
+   int n;
+};
+
 struct Mesh {
    int Nr, Nz, NgRa, NgRb, NgZa, NgZb;
    int nann;          // Nr*Nz annuli
@@ -26,6 +42,8 @@ struct Mesh {
    const double *z_kph;  // index -1 valid
    double Pmax;
    const int *I0;        // [nann] ring start cells of the current substep
+   TileList tiles;       // the cells in storage order
+   TileList etiles;      // the faces of both directions (r, then z) in storage order
 };
 
 // One ring of cells read from its start cell I0: element x (0 <= x <= N) is

@@ -220,11 +220,42 @@ inline std::vector<int> strip_heights(int K)
    return out;
 }
 
+// The tiles of a sequence of groups: `first` and `size` are each group's
+// storage start and element count, `group` and `dim` what its tiles hand to
+// a kernel.
+struct GroupSeq {
+   std::vector<int> first, size, group, dim;
+   void add(int f, int n, int g, int d)
+   {
+      first.push_back(f);
+      size.push_back(n);
+      group.push_back(g);
+      dim.push_back(d);
+   }
+};
+
+template <class X>
+int put_tiles(X &x, TileList &out, const GroupSeq &s)
+{
+   std::vector<Tile> t;
+   for (size_t p = 0; p < s.first.size(); ++p)
+      for (int i = 0; i < s.size[p]; i += TILE)
+         t.push_back({s.first[p] + i, s.size[p] - i < TILE ? s.size[p] - i : TILE, s.group[p],
+                      s.dim[p]});
+   Tile *d = nullptr;
+   DH_TRY(alloc_n(x, &d, sizeof(Tile) * (t.empty() ? 1 : t.size())));
+   if (!t.empty()) DH_TRY(x.put(d, t.data(), sizeof(Tile) * t.size()));
+   out.t = d;
+   out.n = (int)t.size();
+   return DH_OK;
+}
+
 // One group order on the device from the host lists of the visited groups'
 // storage starts and sizes.
 template <class X>
-int put_order(X &x, GroupOrder &o, const std::vector<int> &first, const std::vector<int> &size)
+int put_order(X &x, GroupOrder &o, const GroupSeq &seq)
 {
+   const std::vector<int> &first = seq.first, &size = seq.size;
    int ng = (int)first.size();
    std::vector<int> pos(ng + 1, 0);
    for (int p = 0; p < ng; ++p) pos[p + 1] = pos[p] + size[p];
@@ -246,44 +277,60 @@ int put_order(X &x, GroupOrder &o, const std::vector<int> &first, const std::vec
    o.pos = d[1];
    o.chunk = d[2];
    o.ng = ng;
-   return DH_OK;
+   return put_tiles(x, o.tiles, seq);
 }
 
-// The strip orders of every kind (OrderSet).  fI holds the host copies of
+// The storage-order tiles of the cells and faces and the strip orders of every kind (OrderSet).  fI holds the host copies of
 // both face lists' pair offsets.
 template <class X>
 int build_orders(X &x, Buffers &b, const std::vector<int> *fI)
 {
-   const Mesh &m = b.m;
+   Mesh &m = b.m;
    int Nr = m.Nr, Nz = m.Nz;
-   for (int S : strip_heights(Nz)) {
-      // (j, k) of the cells' groups in this strip order
-      std::vector<std::pair<int, int>> seq;
-      for (int k0 = 0; k0 < Nz; k0 += S)
-         for (int j = 0; j < Nr; ++j)
-            for (int k = k0; k < k0 + S && k < Nz; ++k) seq.push_back({j, k});
-      std::vector<int> first[ORD_KINDS], size[ORD_KINDS];
-      int nfr = fI[0].empty() ? 0 : fI[0].back();
-      for (auto jk : seq) {
+   int nfr = fI[0].empty() ? 0 : fI[0].back();
+   // the sequences of every kind that visit the annuli (j, k) in order
+   auto sequences = [&](const std::vector<std::pair<int, int>> &order, GroupSeq *seq) {
+      for (auto jk : order) {
          int j = jk.first, k = jk.second;
          int a = j + Nr * k;
-         first[ORD_CELLS].push_back(b.h_off[a]);
-         size[ORD_CELLS].push_back(b.h_Np[a]);
+         seq[ORD_CELLS].add(b.h_off[a], b.h_Np[a], a, 0);
          for (int d = 0; d < 2; ++d) {
             int J = d == 0 ? Nr - 1 : Nr, K = d == 0 ? Nz : Nz - 1;
             if (j >= J || k >= K || fI[d].empty()) continue;
             int P = j + J * k;
             int f0 = fI[d][P], nf = fI[d][P + 1] - fI[d][P];
-            first[ORD_FACES_R + d].push_back(f0);
-            size[ORD_FACES_R + d].push_back(nf);
-            first[ORD_EDGES].push_back(d == 0 ? f0 : nfr + f0);
-            size[ORD_EDGES].push_back(nf);
+            seq[ORD_FACES_R + d].add(f0, nf, P, d + 1);
+            seq[ORD_EDGES].add(d == 0 ? f0 : nfr + f0, nf, P, d + 1);
          }
       }
+   };
+   {
+      std::vector<std::pair<int, int>> order;
+      for (int k = 0; k < Nz; ++k)
+         for (int j = 0; j < Nr; ++j) order.push_back({j, k});
+      GroupSeq seq[ORD_KINDS], edges;
+      sequences(order, seq);
+      DH_TRY(put_tiles(x, m.tiles, seq[ORD_CELLS]));
+      for (int d = 0; d < 2; ++d) {
+         const GroupSeq &f = seq[ORD_FACES_R + d];
+         DH_TRY(put_tiles(x, b.F[d].tiles, f));
+         for (size_t p = 0; p < f.first.size(); ++p)
+            edges.add((d == 0 ? 0 : nfr) + f.first[p], f.size[p], f.group[p], d + 1);
+      }
+      if (b.mhd) DH_TRY(put_tiles(x, m.etiles, edges));
+   }
+   for (int S : strip_heights(Nz)) {
+      // (j, k) of the cells' groups in this strip order
+      std::vector<std::pair<int, int>> order;
+      for (int k0 = 0; k0 < Nz; k0 += S)
+         for (int j = 0; j < Nr; ++j)
+            for (int k = k0; k < k0 + S && k < Nz; ++k) order.push_back({j, k});
+      GroupSeq seq[ORD_KINDS];
+      sequences(order, seq);
       for (int kind = 0; kind < ORD_KINDS; ++kind) {
          OrderSet &os = b.ord[kind];
          if (os.n >= MAX_ORDERS) return fail(DH_EINVAL, "too many traversal orders");
-         DH_TRY(put_order(x, os.o[os.n], first[kind], size[kind]));
+         DH_TRY(put_order(x, os.o[os.n], seq[kind]));
          os.strip[os.n] = S;
          ++os.n;
       }

@@ -1,0 +1,58 @@
+"""Meshes whose annuli are long enough for the launches by tiles (at least
+0.94 of the lanes of each annulus's 64-cell tiles at work), and meshes just
+below that, stepped on the GPU and by the host build of the same kernels
+from one state: last tiles of 1 and of 63 cells, whole tiles, and annuli of
+one tile less."""
+import os
+import tempfile
+
+import numpy as np
+import pytest
+
+from disco_amd import capi, configs, state_io
+from disco_amd.host_lib import HostRun
+
+pytestmark = pytest.mark.gpu
+
+
+def _initial(cname, over):
+    cfg = configs.get(cname)
+    par = cfg.par_dict(**over)
+    d = tempfile.mkdtemp(prefix="tiles_")
+    run = HostRun(cname, state_io.write_par(d, dict(par, Autotune=0)))
+    path = os.path.join(d, "init.dstate")
+    run.write(path)
+    run.close()
+    return cfg, par, state_io.read_state(path)
+
+
+# aspect scales the cells per annulus (Np = 2 pi r / (aspect dr))
+@pytest.mark.parametrize("cname,over", [
+    ("euler_yee", {"Num_R": 6, "aspect": 0.02}),       # 314 to 1884 cells
+    ("euler_yee", {"Num_R": 12, "aspect": 0.0982}),    # 64 to 767: the first annulus one full tile
+    ("euler_yee_n1", {"Num_R": 5, "aspect": 0.04, "Riemann_Solver": 0}),
+    ("disk_planet", {"Num_R": 9, "aspect": 0.05}),
+    ("mhd_kep", {"Num_R": 6, "Num_Z": 3, "aspect": 0.03}),
+    ("mhd_kep", {"Num_R": 6, "Num_Z": 3, "aspect": 0.3}),  # below the rule's line
+    ("gr_disk", {"Num_R": 5, "Num_Z": 3, "aspect": 0.05, "R_Min": 8.0, "R_Max": 20.0, "CFL": 0.2,
+                 "Riemann_Solver": 0}),
+])
+def test_long_annuli_step_as_the_host_build(cname, over):
+    import sys
+    sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpu_engine"))
+    import build as cpu_build
+    from helpers import compare_states
+    cfg, par, a = _initial(cname, over)
+    print(f"case {cname} {over}: annuli of {a.np_.min()} to {a.np_.max()} cells", flush=True)
+    gpu = capi.DiscoHip(cfg, par, a)
+    cpu = capi.DiscoHip(cfg, par, a, library=capi.load_library(cpu_build.build()))
+    nvar = 6
+    gpu.autotune(nvar)  # every order of the tiles
+    for _ in range(nvar + 1):
+        dt = min(gpu.getmindt(), 1e-4)
+        gpu.timestep(dt)
+        cpu.timestep(dt)
+    # the parity bar of the GPU against the host build (helpers.PARITY_TOL)
+    print("  worst", compare_states(gpu.download(a), cpu.download(a)), flush=True)
+    gpu.close()
+    cpu.close()
