@@ -462,6 +462,7 @@ int create_buffers(X &x, Buffers &b, const dh_grid *g, const dh_params &P)
    size_t cb = sizeof(double) * (size_t)ntot;
    DH_TRY(alloc_n(x, &b.prim, qb));
    DH_TRY(alloc_n(x, &b.cons, qb));
+   DH_TRY(x.zero(b.cons, qb));  // (nothing writes the ghost cells')
    DH_TRY(alloc_n(x, &b.rkcons, qb));
    DH_TRY(x.zero(b.rkcons, qb));
    DH_TRY(alloc_n(x, &b.gradp, qb));
