@@ -148,7 +148,7 @@ struct Euler {
       double v = P.viscosity;
       if (P.alpha_flag) {
          double c = sqrt(P.gamma_law * prim[PPP] / prim[RHO]);
-         double h = c * pow(r, 1.5);
+         double h = c * pow_3_2(r);
          v = P.viscosity * c * h;
       }
       return v;
@@ -290,8 +290,9 @@ struct Euler {
             Ustr[q] = (aR * Ul[q] + aL * Ur[q] + Fl[q] - Fr[q]) / (aL + aR);
          }
       } else {
-         double Uk[NQ], Fk[NQ];
-         const double *pk = (w < Ss) ? pL : pR;
+         double Uk[NQ], Fk[NQ], pk[NQ];
+#pragma unroll
+         for (int q = 0; q < NQ; ++q) pk[q] = (w < Ss) ? pL[q] : pR[q];
          double Sk = (w < Ss) ? Sl : Sr;
          prim2cons(P, pk, Uk, r, z, 1.0);
          getUstar(P, pk, Ustr, r, Sk, Ss, n);

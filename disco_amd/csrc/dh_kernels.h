@@ -810,6 +810,10 @@ struct KFluxTrans {
 DHD double fgrav(double M, double r, double eps, int type, double n)
 {
    if (type == 0) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      // PHI_ORDER 2 (always, in practice): squares, and one power of 3/2
+      if (n == 2.0) return M * r / pow_3_2(r * r + eps * eps);
+#endif
       return M * pow(r, n - 1.) / pow(pow(r, n) + pow(eps, n), 1. + 1. / n);
    } else if (type == 1) {
       return M / ((r - 2 * M) * (r - 2 * M));
