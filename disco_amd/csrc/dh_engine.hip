@@ -44,9 +44,25 @@ __device__ __forceinline__ unsigned block_of(int xcd)
    return xcd ? (b % NXCD) * (gridDim.x / NXCD) + b / NXCD : b;
 }
 
+// The wavefronts per SIMD a kernel asks the compiler to leave room for (its
+// min_waves member; otherwise whatever its registers allow).
+template <class K, class = void>
+struct MinWaves {
+   static constexpr int value = 1;
+};
+template <class K>
+struct MinWaves<K, decltype((void)K::min_waves)> {
+   static constexpr int value = K::min_waves;
+};
+template <class K1, class K2>
+struct MinWaves<KBoth<K1, K2>> {
+   static constexpr int value =
+       MinWaves<K1>::value > MinWaves<K2>::value ? MinWaves<K1>::value : MinWaves<K2>::value;
+};
+
 // A kernel over cells or faces by elements.
 template <class K>
-__global__ __launch_bounds__(TPB) void k_elems(K k, long n, int xcd)
+__global__ __launch_bounds__(TPB, MinWaves<K>::value) void k_elems(K k, long n, int xcd)
 {
    long t = (long)block_of(xcd) * TPB + threadIdx.x;
    if (t < n) k(t);
@@ -83,6 +99,13 @@ struct ByElements<KBoth<K1, K2>> {
 static bool by_tiles(const TileList &tl, long n) { return n >= 0.94 * 64.0 * tl.n; }
 
 template <class K>
+DHD TileList tiles_of(const K &k) { return k.tiles(); }
+template <class K1, class K2>
+DHD TileList tiles_of(const KBoth<K1, K2> &k)
+{
+   return {nullptr, tiles_of(k.k1).n + tiles_of(k.k2).n};
+}
+template <class K>
 __device__ __forceinline__ void tile_wave(const K &k, const TileList &tl, int w, int lane)
 {
    if (w >= tl.n) return;
@@ -98,16 +121,9 @@ __device__ __forceinline__ void tile_wave(const K &k, const TileList &tl, int w,
 template <class K1, class K2>
 __device__ __forceinline__ void tile_wave(const KBoth<K1, K2> &k, const TileList &, int w, int lane)
 {
-   TileList a = k.k1.tiles();
+   TileList a = tiles_of(k.k1);
    if (w < a.n) tile_wave(k.k1, a, w, lane);
-   else tile_wave(k.k2, k.k2.tiles(), w - a.n, lane);
-}
-template <class K>
-DHD TileList tiles_of(const K &k) { return k.tiles(); }
-template <class K1, class K2>
-DHD TileList tiles_of(const KBoth<K1, K2> &k)
-{
-   return {nullptr, tiles_of(k.k1).n + tiles_of(k.k2).n};
+   else tile_wave(k.k2, tiles_of(k.k2), w - a.n, lane);
 }
 constexpr int WAVES = TPB / 64;
 __device__ __forceinline__ int wave_of(unsigned blk)
@@ -190,31 +206,109 @@ __global__ __launch_bounds__(TPB) void k_ring_start(Mesh m, const double *piph, 
    ring_start_block(m, piph, I0, blockIdx.x);
 }
 
-// flip_fluxes (bfields.c:742-814): one wavefront per face track; the lanes
-// read 64 flags at a time and lane 0 hands the flagged faces over in order.
-__device__ __forceinline__ void flips_block(const Mesh &m, int dim, const Faces &F, const signed char *flag,
-                            double *Phi, double *rkPhi, unsigned blk)
+// check_flipped and flip_fluxes (bfields.c:693-814): one workgroup per face
+// track takes TPB faces at a time, each thread the flag of one face, and
+// hands the flagged faces over.  A flip of face n reads and writes fluxes of
+// faces n - 1, n and n + 1, in slots of these faces' cells (a face whose
+// owner changed names its other cell's slot from then on), and owners of
+// n - 1 and n.  So two consecutive flagged faces p < b are independent when
+// faces p + 1 and b - 1 share no cell: the batch's flagged faces fall into
+// runs, each run's first thread hands its run over in order, all runs at
+// once.  The result is the reference's face-by-face order: batches are in
+// order, and where a track of one batch closes on itself its last run waits
+// for the first unless those two share no cell either.  The flags are those
+// of the owners before any flip: of the faces of a later batch only the
+// last one of the track can have changed owner (by a flip of face 0), so its
+// position is kept from the start.
+//
+// What bounds it: a chain of two loads and the longest run.  Flags in
+// launches of their own and one lane per track handing over its whole track
+// took 2 x (8 + 49) us a step on the 32 x 8 disk, whose shear flips most faces;
+// now 97.
+template <int DIM>
+__device__ __forceinline__ void flip_track(const Mesh &m, const Faces &F, const double *piph,
+                                           const double *wiph, double dt, double *Phi,
+                                           double *rkPhi, int JK)
 {
-   int JK = blk * (TPB / 64) + threadIdx.x / 64;
-   int lane = threadIdx.x & 63;
-   if (JK >= F.npairs || track_skipped(F.npairs, JK)) return;
-   int base = F.fI[JK], N = F.fI[JK + 1] - base;
-   for (int chunk = 0; chunk < N; chunk += 64) {
-      int n = chunk + lane;
-      unsigned long long bits = __ballot(n < N && flag[base + n] != 0);
-      if (lane == 0) {
-         while (bits) {
-            int b = __ffsll((long long)bits) - 1;
-            bits &= bits - 1;
-            flip_one(dim, (size_t)m.ntot, F, base, N, chunk + b, Phi, rkPhi);
-         }
+   __shared__ double s_up[TPB + 1];  // moved upper edges: [0] the face before the batch
+   __shared__ unsigned long long s_flag[WAVES], s_start[WAVES];
+   if (track_skipped(F.npairs, JK)) return;
+   const int base = F.fI[JK], N = F.fI[JK + 1] - base;
+   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+   KFlipFlags<DIM> k{m, F, piph, wiph, &dt, nullptr};
+   // whether faces f and g of the track (0 <= f, g < N) share a cell
+   auto share = [&](int f, int g) {
+      return F.L[base + f] == F.L[base + g] || F.R[base + f] == F.R[base + g];
+   };
+   // the next bit at or after i, and the last one before i (-1: none)
+   auto next_bit = [&](const unsigned long long *b, int i) {
+      for (int w = i >> 6; w < WAVES; ++w) {
+         unsigned long long x = b[w];
+         if (w == i >> 6) x &= ~0ULL << (i & 63);
+         if (x) return 64 * w + __ffsll((long long)x) - 1;
+      }
+      return TPB;
+   };
+   auto last_bit = [&](const unsigned long long *b, int i) {
+      for (int w = (i - 1) >> 6; w >= 0 && i > 0; --w) {
+         unsigned long long x = b[w];
+         if (w == i >> 6) x &= (1ULL << (i & 63)) - 1;
+         if (x) return 64 * w + 63 - __clzll((long long)x);
+      }
+      return -1;
+   };
+   const double last = k.moved_up(base + N - 1);
+   for (int n0 = 0; n0 < N; n0 += TPB) {
+      const int n = n0 + tid;
+      double up = 0.0;
+      if (n < N) up = n == N - 1 ? last : k.moved_up(base + n);
+      double prev = n0 == 0 ? last : s_up[TPB];  // (the last batch's final edge)
+      __syncthreads();
+      if (tid == 0) s_up[0] = prev;
+      s_up[tid + 1] = up;
+      __syncthreads();
+      bool flag = n < N && get_sdp(up, s_up[tid], m.Pmax) < 0.;
+      unsigned long long b = __ballot(flag);
+      if (lane == 0) s_flag[wv] = b;
+      if (!__syncthreads_or(flag)) continue;
+      bool start = false;
+      if (flag) {
+         int p = last_bit(s_flag, tid);
+         start = p < 0 || (tid - p > 2 && !share(n0 + p + 1, n - 1));
+      }
+      b = __ballot(start);
+      if (lane == 0) s_start[wv] = b;
+      __syncthreads();
+      int end = start ? next_bit(s_start, tid + 1) : tid;
+      bool wait = false;
+      if (start && N <= TPB && end == TPB) {  // the last run of a one-batch track
+         int l = next_bit(s_flag, 0), h = last_bit(s_flag, TPB);
+         if (next_bit(s_start, 0) != tid)  // (a single run has nothing to wait for)
+            wait = l + N - h <= 2 || share((h + 1) % N, (l + N - 1) % N);
+      }
+      for (int phase = 0; phase < 2; ++phase) {
+         if (start && wait == (phase == 1))
+            for (int i = tid; i < end; i = next_bit(s_flag, i + 1))
+               flip_one(DIM, (size_t)m.ntot, F, base, N, n0 + i, Phi, rkPhi);
+         __syncthreads();
       }
    }
 }
-__global__ __launch_bounds__(TPB) void k_flips(Mesh m, int dim, Faces F, const signed char *flag,
-                                               double *Phi, double *rkPhi)
+// The tracks of both directions (they share no flux slot): the r tracks,
+// then the z tracks.
+__device__ __forceinline__ void flips_block(const Mesh &m, const Faces &Fr, const Faces &Fz,
+                                            const double *piph, const double *wiph, double dt,
+                                            double *Phi, double *rkPhi, unsigned blk)
 {
-   flips_block(m, dim, F, flag, Phi, rkPhi, blockIdx.x);
+   int nr = Fr.npairs;
+   if ((int)blk < nr) flip_track<1>(m, Fr, piph, wiph, dt, Phi, rkPhi, (int)blk);
+   else flip_track<2>(m, Fz, piph, wiph, dt, Phi, rkPhi, (int)blk - nr);
+}
+__global__ __launch_bounds__(TPB) void k_flips(Mesh m, Faces Fr, Faces Fz, const double *piph,
+                                               const double *wiph, const double *dtp, double *Phi,
+                                               double *rkPhi)
+{
+   flips_block(m, Fr, Fz, piph, wiph, *dtp, Phi, rkPhi, blockIdx.x);
 }
 
 // The ghost-ring walk (KBcScan), one workgroup per ring.  The walk's state
@@ -277,10 +371,47 @@ __device__ __forceinline__ void bc_scan_block(const Mesh &m, int side, const dou
    __syncthreads();
    if (s_miss && tid == 0) KBcScan{m, side, piph, dphi, start}(t);
 }
-__global__ __launch_bounds__(TPB) void k_bc_scan(Mesh m, int side, const double *piph,
-                                                 const double *dphi, int *start)
+// The ghost rings of a direction's sides (r or z; at most two, which share no
+// annulus they write): every ring of every side in one launch, then one
+// workgroup per line of a side that fills its layers from the innermost out
+// (a layer copies from the one inside it, of the same line).  A launch per
+// side and layer made 12 launches a step of the MHD disks, most of them
+// shorter than the gap to the next: 83 us a step on the 32 x 8 disk, now 39.
+__device__ __forceinline__ void bc_rings_block(const Mesh &m, const BcSides &s, const double *piph,
+                                               const double *dphi, int *start, unsigned blk)
 {
-   bc_scan_block(m, side, piph, dphi, start, blockIdx.x);
+   unsigned r0 = (unsigned)(s.lines[0] * s.layers[0]);
+   int i = blk < r0 ? 0 : 1;
+   bc_scan_block(m, s.side[i], piph, dphi, start, i == 0 ? blk : blk - r0);
+}
+template <int NQ>
+__device__ __forceinline__ void bc_columns_block(const Mesh &m, const BcSides &s,
+                                                 const int *start, double *prim,
+                                                 const double *piph, const double *dphi,
+                                                 unsigned blk)
+{
+   int i = (int)blk < s.lines[0] ? 0 : 1;
+   int line = i == 0 ? (int)blk : (int)blk - s.lines[0];
+   for (int g = 0; g < s.layers[i]; ++g) {
+      KBcFill<NQ> k{m, s.side[i], g, s.diode[i], start, prim, piph, dphi, 0};
+      int dst, src;
+      bc_pair(m, s.side[i], line, g, &dst, &src);
+      for (int c = threadIdx.x; c < m.Np[dst]; c += blockDim.x) k.cell(line, c);
+      __syncthreads();  // the next layer reads this one
+   }
+}
+__global__ __launch_bounds__(TPB) void k_bc_rings(Mesh m, BcSides s, const double *piph,
+                                                  const double *dphi, int *start)
+{
+   bc_rings_block(m, s, piph, dphi, start, blockIdx.x);
+}
+constexpr int BC_TPB = 1024;
+template <int NQ>
+__global__ __launch_bounds__(BC_TPB) void k_bc_columns(Mesh m, BcSides s, const int *start,
+                                                       double *prim, const double *piph,
+                                                       const double *dphi)
+{
+   bc_columns_block<NQ>(m, s, start, prim, piph, dphi, blockIdx.x);
 }
 
 // add_diagnostics (analysis.c:52-106): one workgroup per annulus; each
@@ -717,24 +848,32 @@ struct HipExec {
       return DH_OK;
    }
 
-   int bc_scan(const Mesh &m, int side, const double *piph, const double *dphi, int *start)
+   template <int NQ>
+   int ghost_rings(const Mesh &m, const BcSides &s, const double *piph, const double *dphi,
+                   int *start, double *prim)
    {
-      long rings = (long)bc_lines(m, side) * bc_layers(m, side);
-      if (rings <= 0) return DH_OK;
+      if (s.rings() == 0) return DH_OK;
       {
          Bracket b(*this, "bc_scan");
-         k_bc_scan<<<(unsigned)rings, TPB, 0, stream>>>(m, side, piph, dphi, start);
+         k_bc_rings<<<s.rings(), TPB, 0, stream>>>(m, s, piph, dphi, start);
+      }
+      LAUNCH_CHECK();
+      {
+         Bracket b(*this, "bc_fill");
+         k_bc_columns<NQ><<<s.columns(), BC_TPB, 0, stream>>>(m, s, start, prim, piph, dphi);
       }
       LAUNCH_CHECK();
       return DH_OK;
    }
 
-   int flips(const Mesh &m, int dim, const Faces &F, const signed char *flag, double *Phi,
-             double *rkPhi)
+   int flip_tracks(const Mesh &m, const Faces &Fr, const Faces &Fz, const double *piph,
+                   const double *wiph, const double *dtp, double *Phi, double *rkPhi)
    {
+      unsigned nb = (unsigned)(Fr.npairs + Fz.npairs);
+      if (nb == 0) return DH_OK;
       {
          Bracket b(*this, "flips");
-         k_flips<<<(unsigned)((F.npairs + 3) / 4), TPB, 0, stream>>>(m, dim, F, flag, Phi, rkPhi);
+         k_flips<<<nb, TPB, 0, stream>>>(m, Fr, Fz, piph, wiph, dtp, Phi, rkPhi);
       }
       LAUNCH_CHECK();
       return DH_OK;
@@ -1001,6 +1140,7 @@ static int do_faces(dh_ctx *c)
 // ---------------------------------------------------------------------------
 template <class K>
 struct RunOp {
+   static constexpr int min_waves = MinWaves<K>::value;
    K k;
    long n;
    unsigned blocks() const { return nblocks(n); }
@@ -1013,6 +1153,7 @@ struct RunOp {
 // A kernel over cells or faces by tiles.
 template <class K>
 struct TileOp {
+   static constexpr int min_waves = 1;
    K k;
    unsigned blocks() const { return nblocks((long)tiles_of(k).n * 64); }
    __device__ __forceinline__ void run(unsigned b) const
@@ -1021,6 +1162,7 @@ struct TileOp {
    }
 };
 struct RingStartOp {
+   static constexpr int min_waves = 1;
    Mesh m;
    const double *piph;
    int *I0;
@@ -1028,24 +1170,46 @@ struct RingStartOp {
    __device__ __forceinline__ void run(unsigned b) const { ring_start_block(m, piph, I0, b); }
 };
 struct FlipsOp {
+   static constexpr int min_waves = 1;
    Mesh m;
-   int dim;
-   Faces F;
-   const signed char *flag;
+   Faces Fr, Fz;
+   const double *piph, *wiph, *dtp;
    double *Phi, *rkPhi;
-   unsigned blocks() const { return (unsigned)((F.npairs + 3) / 4); }
-   __device__ __forceinline__ void run(unsigned b) const { flips_block(m, dim, F, flag, Phi, rkPhi, b); }
+   unsigned blocks() const { return (unsigned)(Fr.npairs + Fz.npairs); }
+   __device__ __forceinline__ void run(unsigned b) const
+   {
+      flips_block(m, Fr, Fz, piph, wiph, *dtp, Phi, rkPhi, b);
+   }
 };
-struct BcScanOp {
+struct BcRingsOp {
+   static constexpr int min_waves = 1;
    Mesh m;
-   int side;
+   BcSides s;
    const double *piph, *dphi;
    int *start;
-   unsigned blocks() const { return (unsigned)((long)bc_lines(m, side) * bc_layers(m, side)); }
-   __device__ __forceinline__ void run(unsigned b) const { bc_scan_block(m, side, piph, dphi, start, b); }
+   unsigned blocks() const { return s.rings(); }
+   __device__ __forceinline__ void run(unsigned b) const
+   {
+      bc_rings_block(m, s, piph, dphi, start, b);
+   }
+};
+template <int NQ>
+struct BcColumnsOp {
+   static constexpr int min_waves = 1;
+   Mesh m;
+   BcSides s;
+   const int *start;
+   double *prim;
+   const double *piph, *dphi;
+   unsigned blocks() const { return s.columns(); }
+   __device__ __forceinline__ void run(unsigned b) const
+   {
+      bc_columns_block<NQ>(m, s, start, prim, piph, dphi, b);
+   }
 };
 template <int NQ, class H>
 struct MindtOp {
+   static constexpr int min_waves = 1;
    Mesh m;
    dh_params P;
    const double *prim, *piph, *dphi, *wiph;
@@ -1064,6 +1228,7 @@ struct EnsDiagArgs {
 };
 template <int KIND>
 struct DiagOp {
+   static constexpr int min_waves = 1;
    Mesh m;
    dh_params P;
    const EnsDiagArgs *a;
@@ -1080,7 +1245,7 @@ struct DiagOp {
 // finds it; a bisection of the meshes' block offsets was a chain of four to
 // six dependent loads at the head of every workgroup.
 template <class Op>
-__global__ __launch_bounds__(TPB) void k_group(const Op *__restrict__ ops,
+__global__ __launch_bounds__(TPB, Op::min_waves) void k_group(const Op *__restrict__ ops,
                                                const int2 *__restrict__ map)
 {
    int2 e = map[blockIdx.x];
@@ -1155,16 +1320,19 @@ struct GroupExec {
    {
       return rec(RingStartOp{m, piph, I0});
    }
-   int bc_scan(const Mesh &m, int side, const double *piph, const double *dphi, int *start)
+   template <int NQ>
+   int ghost_rings(const Mesh &m, const BcSides &s, const double *piph, const double *dphi,
+                   int *start, double *prim)
    {
-      if ((long)bc_lines(m, side) * bc_layers(m, side) <= 0) return DH_OK;
-      return rec(BcScanOp{m, side, piph, dphi, start});
+      if (s.rings() == 0) return DH_OK;
+      DH_TRY(rec(BcRingsOp{m, s, piph, dphi, start}));
+      return rec(BcColumnsOp<NQ>{m, s, start, prim, piph, dphi});
    }
-   int flips(const Mesh &m, int dim, const Faces &F, const signed char *flag, double *Phi,
-             double *rkPhi)
+   int flip_tracks(const Mesh &m, const Faces &Fr, const Faces &Fz, const double *piph,
+                   const double *wiph, const double *dtp, double *Phi, double *rkPhi)
    {
-      if (F.npairs <= 0) return DH_OK;
-      return rec(FlipsOp{m, dim, F, flag, Phi, rkPhi});
+      if (Fr.npairs + Fz.npairs <= 0) return DH_OK;
+      return rec(FlipsOp{m, Fr, Fz, piph, wiph, dtp, Phi, rkPhi});
    }
    template <int NQ>
    int c2p_guess(const Mesh &, const dh_params &, const double *, const double *, const double *,

@@ -652,6 +652,7 @@ template <int NQ, class H>
 struct KFluxPhi {
    Mesh m;
    static constexpr bool by_elements = true;  // bound by its arithmetic: no lane to spare
+   static constexpr int min_waves = IsGR<H>::value ? 2 : 1;  // of the relativistic HLLD's registers
    dh_params P;
    const double *dtp;
    const double *prim, *gradp, *gradr, *gradz, *piph, *dphi, *wiph;
@@ -727,6 +728,7 @@ template <int NQ, class H, int DIM>
 struct KFluxTrans {
    Mesh m;
    static constexpr bool by_elements = true;
+   static constexpr int min_waves = IsGR<H>::value ? 2 : 1;  // of the relativistic HLLD's registers
    dh_params P;
    static constexpr int dim = DIM;
    const double *dtp;
@@ -1830,6 +1832,23 @@ DHD int bc_layers(const Mesh &m, int side)
    return side == 0 ? m.NgRa : side == 1 ? m.NgRb : side == 2 ? m.NgZa : m.NgZb;
 }
 
+// The sides of one direction (r or z) whose ghost annuli are copied.
+struct BcSides {
+   int n, side[2], diode[2], lines[2], layers[2];
+   DHD unsigned rings() const
+   {
+      unsigned r = 0;
+      for (int i = 0; i < n; ++i) r += (unsigned)(lines[i] * layers[i]);
+      return r;
+   }
+   DHD unsigned columns() const
+   {
+      unsigned r = 0;
+      for (int i = 0; i < n; ++i) r += (unsigned)lines[i];
+      return r;
+   }
+};
+
 // Overlap in phi of destination cell (phim, phip] with source cell i1,
 // shifted by whole periods next to it as the reference does; returns the
 // shifted upper edge of the source cell.
@@ -1935,10 +1954,11 @@ struct KBcFill {
    double *prim;
    const double *piph, *dphi;
    int maxnp;  // cells per line slot: the largest Np of the layer's annuli
-   DHD void operator()(long t) const
+   DHD void operator()(long t) const { cell((int)(t / maxnp), (int)(t % maxnp)); }
+   // cell i of a line's ghost ring (nothing where the ring is shorter)
+   DHD void cell(int line, int i) const
    {
       size_t nt = (size_t)m.ntot;
-      int line = (int)(t / maxnp), i = (int)(t % maxnp);
       int dst, src;
       bc_pair(m, side, line, g, &dst, &src);
       int Np = m.Np[dst];

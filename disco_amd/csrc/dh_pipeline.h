@@ -7,7 +7,11 @@
 // against the oracle.  X provides
 //   run(name, kernel, n)          kernel(t) for t in [0, n)
 //   ring_start(m, piph, I0)       start cell of every annulus
-//   flips(m, dim, F, flag, Phi, rkPhi)   hand-overs of flagged faces per track
+//   flip_tracks(m, Fr, Fz, piph, wiph, dtp, Phi, rkPhi)   flags and hand-overs of
+//                                 every track's flipped faces; or
+//   flips(m, dim, F, flag, Phi, rkPhi)   the hand-overs alone, of flagged faces
+//   ghost_rings<NQ>(m, sides, piph, dphi, start, prim)   the copied ghost annuli of a
+//                                 direction; or bc_scan and KBcFill, side by side
 //   min_dt<NQ,H>(m, P, prim, piph, dphi, wiph, &dt)
 //   diag(m, P, kind, pl1, prim, piph, dphi, dt, Qrz)   per-annulus diagnostics
 //   c2p_guess<NQ>(m, P, cons, piph, dphi, prm, frag, guess)   learned cons2prim guesses
@@ -91,7 +95,6 @@ struct Buffers {
    int *bcstart = nullptr;          // where each ghost cell's overlap sum starts
    // Traversal orders the executor may launch a kernel in (OrderSet)
    OrderSet ord[ORD_KINDS];
-   OrderSet none;  // storage order only (launches whose elements are not one kind)
    int bc_maxnp[4][8] = {{0}};      // largest Np of each side's ghost layers
    PlanetSet pl[2];
    StepArgs *step = nullptr;  // device copy of {dt, planets} of the current timestep
@@ -346,6 +349,36 @@ int run_ord(X &x, const char *name, const K &k, long n, const OrderSet &os)
    return x.run_tuned(name, k, n, os.o, os.n, os.strip);
 }
 
+// Two kernels that share no data as one launch, k1 over n1 elements and k2
+// over n2.
+template <class X, class K1, class K2>
+int run_both(X &x, const char *name, const K1 &k1, long n1, const K2 &k2, long n2)
+{
+   return x.run_tuned(name, KBoth<K1, K2>{k1, k2, n1}, n1 + n2, nullptr, 0, nullptr);
+}
+
+// Whether an executor flags and hands over the flipped faces of every track
+// in one launch (flip_tracks) rather than by KFlipFlags and flips.
+template <class X, class = void>
+struct HasFlipTracks {
+   static constexpr bool value = false;
+};
+template <class X>
+struct HasFlipTracks<X, decltype((void)&X::flip_tracks)> {
+   static constexpr bool value = true;
+};
+
+// Whether an executor walks and fills the ghost rings of a direction's two
+// sides together (ghost_rings).
+template <class X, class = void>
+struct HasGhostRings {
+   static constexpr bool value = false;
+};
+template <class X>
+struct HasGhostRings<X, decltype((void)&X::template ghost_rings<5>)> {
+   static constexpr bool value = true;
+};
+
 // Allocates and fills every buffer of a validated mesh.
 template <class X>
 int create_buffers(X &x, Buffers &b, const dh_grid *g, const dh_params &P)
@@ -437,7 +470,7 @@ int create_buffers(X &x, Buffers &b, const dh_grid *g, const dh_params &P)
       DH_TRY(alloc_n(x, &b.rng[d], sizeof(int) * 2 * (size_t)ntot));
       if (b.mhd) {
          DH_TRY(alloc_n(x, &b.emf_f[d], sizeof(double) * 3 * n));
-         DH_TRY(alloc_n(x, &b.flag[d], sizeof(signed char) * n));
+         if (!HasFlipTracks<X>::value) DH_TRY(alloc_n(x, &b.flag[d], sizeof(signed char) * n));
          DH_TRY(alloc_n(x, &b.estep[d], sizeof(int) * 2 * n));
          // edge lines: the line whose first list is pair P holds the merge
          // of P's faces with the next pair's (r faces: k + 1, z faces: j + 1)
@@ -548,6 +581,7 @@ struct Engine {
       const Mesh &m = b.m;
       if (!dim_active(m, 1) && !dim_active(m, 2)) return DH_OK;
       if (!reuse) DH_TRY(x.ring_start(m, b.piph, b.I0));
+      if (merged() && dim_active(m, 1) && dim_active(m, 2)) return topology_merged<NQ>(grads, reuse);
       for (int dim = 1; dim <= 2; ++dim) {
          int d = dim - 1;
          if (!dim_active(m, dim)) continue;
@@ -580,6 +614,37 @@ struct Engine {
       return DH_OK;
    }
 
+   // Whether launches that share no data go as one: on small meshes, where
+   // every launch waits mostly on its own latency (a dependent launch costs
+   // 5 us and more however little it does).  Above 2^20 cells a launch fills
+   // the card by itself and the merged kernels' registers only cost waves.
+   bool merged() const { return x.merges_launches() && b.m.ntot < SMALL_MESH_CELLS; }
+
+   // The same with the r and the z direction's launches as one.
+   template <int NQ>
+   int topology_merged(bool grads, bool reuse)
+   {
+      const Mesh &m = b.m;
+      if (!reuse) {
+         KCellRanges<1> r1{m, b.piph, b.rng[0]};
+         KCellRanges<2> r2{m, b.piph, b.rng[1]};
+         DH_TRY(run_both(x, "ranges", r1, m.ntot, r2, m.ntot));
+         KFaces<1> f1{m, b.F[0], b.rng[0], b.piph, b.dphi};
+         KFaces<2> f2{m, b.F[1], b.rng[1], b.piph, b.dphi};
+         DH_TRY(run_both(x, "faces", f1, m.ntot, f2, m.ntot));
+      }
+      if (!grads) return DH_OK;
+      if (b.P.plm == 0.0) {
+         DH_TRY(x.zero(b.gradr, sizeof(double) * NQ * m.ntot));
+         return x.zero(b.gradz, sizeof(double) * NQ * m.ntot);
+      }
+      KGrad<NQ, 1> g1{m, b.P.plm, b.P.num_c, b.F[0], b.rng[0], b.piph, b.dphi, b.prim, b.gradp,
+                      b.gradr};
+      KGrad<NQ, 2> g2{m, b.P.plm, b.P.num_c, b.F[1], b.rng[1], b.piph, b.dphi, b.prim, b.gradp,
+                      b.gradz};
+      return run_both(x, "grad", g1, m.ntot, g2, m.ntot);
+   }
+
    // Zero-gradient / diode ghost annuli (onestep.c:194-210): r sides, then z.
    template <int NQ>
    int boundaries()
@@ -587,17 +652,35 @@ struct Engine {
       const Mesh &m = b.m;
       const dh_params &P = b.P;
       int bcs[4] = {P.bc_rmin, P.bc_rmax, P.bc_zmin, P.bc_zmax};
-      for (int side = 0; side < 4; ++side) {
-         if (side >= 2 && m.Nz <= 1) continue;
-         if (bcs[side] != DH_BC_ZEROGRAD && bcs[side] != DH_BC_DIODE) continue;
-         int lines = bc_lines(m, side), layers = bc_layers(m, side);
-         if (layers == 0) continue;
-         DH_TRY(x.bc_scan(m, side, b.piph, b.dphi, b.bcstart));
-         for (int g = 0; g < layers; ++g) {
-            int maxnp = b.bc_maxnp[side][g];
-            KBcFill<NQ> k{m, side, g, bcs[side] == DH_BC_DIODE ? 1 : 0, b.bcstart, b.prim,
-                          b.piph, b.dphi, maxnp};
-            DH_TRY(x.run("bc_fill", k, (long)lines * maxnp));
+      if constexpr (HasGhostRings<X>::value) {
+         for (int dir = 0; dir < 2; ++dir) {
+            if (dir == 1 && m.Nz <= 1) continue;
+            BcSides s;
+            memset(&s, 0, sizeof s);
+            for (int side = 2 * dir; side < 2 * dir + 2; ++side) {
+               if (bcs[side] != DH_BC_ZEROGRAD && bcs[side] != DH_BC_DIODE) continue;
+               if (bc_layers(m, side) == 0) continue;
+               s.side[s.n] = side;
+               s.diode[s.n] = bcs[side] == DH_BC_DIODE;
+               s.lines[s.n] = bc_lines(m, side);
+               s.layers[s.n] = bc_layers(m, side);
+               ++s.n;
+            }
+            DH_TRY(x.template ghost_rings<NQ>(m, s, b.piph, b.dphi, b.bcstart, b.prim));
+         }
+      } else {
+         for (int side = 0; side < 4; ++side) {
+            if (side >= 2 && m.Nz <= 1) continue;
+            if (bcs[side] != DH_BC_ZEROGRAD && bcs[side] != DH_BC_DIODE) continue;
+            int lines = bc_lines(m, side), layers = bc_layers(m, side);
+            if (layers == 0) continue;
+            DH_TRY(x.bc_scan(m, side, b.piph, b.dphi, b.bcstart));
+            for (int g = 0; g < layers; ++g) {
+               int maxnp = b.bc_maxnp[side][g];
+               KBcFill<NQ> k{m, side, g, bcs[side] == DH_BC_DIODE ? 1 : 0, b.bcstart, b.prim,
+                             b.piph, b.dphi, maxnp};
+               DH_TRY(x.run("bc_fill", k, (long)lines * maxnp));
+            }
          }
       }
       return DH_OK;
@@ -622,15 +705,16 @@ struct Engine {
       constexpr bool mhd = IsMHD<H>::value;
       const Mesh &m = b.m;
       const dh_params &P = b.P;
-      // On small meshes, where every launch waits mostly on its own
-      // latency, launches that share no data go as one: the mesh velocity
-      // (wiph) with the phi slopes (gradp), the phi with the r fluxes.
-      const bool merge = x.merges_launches() && m.ntot < SMALL_MESH_CELLS;
+      // The launches that go as one on small meshes (merged()): the mesh
+      // velocity (wiph) with the phi slopes (gradp), the directions of one
+      // kernel, the conserved update with the edge EMFs it shares no data
+      // with, the magnetic fluxes with the edge segments.
+      const bool merge = merged();
+      const bool both = merge && dim_active(m, 1) && dim_active(m, 2);
       KWcell<NQ, H> kw{m, P, b.prim, b.wiph};
       KPlmPhi<NQ> kpl{m, P.plm, b.prim, b.dphi, b.gradp};
       if (first_step && merge && P.mesh_motion != 3) {
-         DH_TRY(run_ord(x, "wcell_plm_phi", KBoth<KWcell<NQ, H>, KPlmPhi<NQ>>{kw, kpl, m.ntot},
-                        2 * m.ntot, b.none));
+         DH_TRY(run_both(x, "wcell_plm_phi", kw, m.ntot, kpl, m.ntot));
       } else {
          if (first_step) {
             DH_TRY(run_ord(x, "wcell", kw, m.ntot, b.ord[ORD_CELLS]));
@@ -641,58 +725,72 @@ struct Engine {
       DH_TRY(topology<NQ>(true, reuse));
       KFluxPhi<NQ, H> kp{m, P, dt, b.prim, b.gradp, b.gradr, b.gradz, b.piph, b.dphi, b.wiph,
                          b.dFp, b.emf_phi};
-      const bool merge_flux = merge && dim_active(m, 1);
-      if (!merge_flux) DH_TRY(run_ord(x, "flux_phi", kp, m.ntot, b.ord[ORD_CELLS]));
-      for (int dim = 1; dim <= 2; ++dim) {
-         int d = dim - 1;
-         if (!dim_active(m, dim)) continue;
-         if (dim == 1) {
-            KFluxTrans<NQ, H, 1> kt{m, P, dt, b.F[d], b.prim, b.gradp, b.gradr, b.gradz,
-                                    b.piph, b.dphi, b.dF[d], b.emf_f[d]};
-            if (merge_flux)
-               DH_TRY(run_ord(x, "flux_phi_r",
-                              KBoth<KFluxPhi<NQ, H>, KFluxTrans<NQ, H, 1>>{kp, kt, m.ntot},
-                              m.ntot + b.F[d].n, b.none));
-            else
-               DH_TRY(run_ord(x, "flux_r", kt, b.F[d].n, b.ord[ORD_FACES_R]));
-         } else {
-            KFluxTrans<NQ, H, 2> kt{m, P, dt, b.F[d], b.prim, b.gradp, b.gradr, b.gradz,
-                                    b.piph, b.dphi, b.dF[d], b.emf_f[d]};
-            DH_TRY(run_ord(x, "flux_z", kt, b.F[d].n, b.ord[ORD_FACES_Z]));
-         }
+      KFluxTrans<NQ, H, 1> kt1{m, P, dt, b.F[0], b.prim, b.gradp, b.gradr, b.gradz, b.piph, b.dphi,
+                               b.dF[0], b.emf_f[0]};
+      KFluxTrans<NQ, H, 2> kt2{m, P, dt, b.F[1], b.prim, b.gradp, b.gradr, b.gradz, b.piph, b.dphi,
+                               b.dF[1], b.emf_f[1]};
+      if (both) {
+         KBoth<KFluxTrans<NQ, H, 1>, KFluxTrans<NQ, H, 2>> kt{kt1, kt2, b.F[0].n};
+         DH_TRY(run_both(x, "flux", kp, m.ntot, kt, (long)b.F[0].n + b.F[1].n));
+      } else if (merge && dim_active(m, 1)) {
+         DH_TRY(run_both(x, "flux_phi_r", kp, m.ntot, kt1, b.F[0].n));
+      } else {
+         DH_TRY(run_ord(x, "flux_phi", kp, m.ntot, b.ord[ORD_CELLS]));
+         if (dim_active(m, 1)) DH_TRY(run_ord(x, "flux_r", kt1, b.F[0].n, b.ord[ORD_FACES_R]));
       }
-      if (mhd) {
-         int ct = P.ct;
-         KEdgesCollect kc{m, ct, b.dphi, b.emf_phi, b.F[0], b.F[1], b.rng[0], b.rng[1],
-                          b.emf_f[0], b.emf_f[1], b.Ecarry, b.Epre};
-         DH_TRY(run_ord(x, "edges_collect", kc, m.ntot, b.ord[ORD_CELLS]));
-         EdgeArgs ea{m, b.F[0], b.F[1], b.rng[0], b.rng[1], b.Epre, b.piph, b.dphi};
-         KEdgesFinal kef{ea, ct, b.wiph, b.emf_f[0], b.emf_f[1], b.Eo, b.Eown, b.Ecarry};
-         DH_TRY(run_ord(x, "edges_final", kef, m.ntot, b.ord[ORD_CELLS]));
-         KUpdateB kb{m, RK, dt, b.F[0], b.F[1], b.rng[0], b.rng[1], b.Eo, st.pin, st.prk, st.pout};
-         DH_TRY(run_ord(x, "update_B", kb, m.ntot, b.ord[ORD_CELLS]));
-         if (dim_active(m, 2)) {
-            if (dim_active(m, 1) && !reuse)
-               DH_TRY(run_ord(x, "line_steps_r", KLineSteps<1>{m, b.F[0], b.estep[0]}, b.F[0].n,
-                              b.ord[ORD_FACES_R]));
-            if (!reuse)
-               DH_TRY(run_ord(x, "line_steps_z", KLineSteps<2>{m, b.F[1], b.estep[1]}, b.F[1].n,
-                              b.ord[ORD_FACES_Z]));
-            KEdgeSegments ks{m, dt, b.F[0], b.F[1], b.estep[0], b.estep[1], b.lbase[0], b.lbase[1],
-                             b.piph, b.dphi, b.Eown, b.seg[0], b.seg[1]};
-            DH_TRY(run_ord(x, "edge_segments", ks, (long)b.F[0].n + b.F[1].n, b.ord[ORD_EDGES]));
-            KEdgeAdjust ke{m, b.F[0], b.F[1], b.estep[0], b.estep[1], b.lbase[0], b.lbase[1],
-                           b.seg[0], b.seg[1], st.pout};
-            DH_TRY(run_ord(x, "edge_adjust", ke, (long)b.F[0].n + b.F[1].n, b.ord[ORD_EDGES]));
-         }
-      }
+      if (!both && dim_active(m, 2))
+         DH_TRY(run_ord(x, "flux_z", kt2, b.F[1].n, b.ord[ORD_FACES_Z]));
       KUpdate<NQ, H> ku{m, P, RK, dt, first_step, &b.step->pl[sub], b.prim, b.prim, st.cin,
                         st.cout, st.crk, b.gradr, b.gradp, b.gradz, b.piph, b.dphi, b.wiph,
                         b.piph2, b.dphi2, b.dFp, b.dF[0], b.dF[1], b.F[0].fI, b.F[1].fI,
                         b.rng[0], b.rng[1], b.F[0].n, b.F[1].n};
-      DH_TRY(run_ord(x, "update", ku, m.ntot, b.ord[ORD_CELLS]));
-      if (mhd) {
-         if (first_step) {
+      if constexpr (mhd) {
+         int ct = P.ct;
+         KEdgesCollect kc{m, ct, b.dphi, b.emf_phi, b.F[0], b.F[1], b.rng[0], b.rng[1],
+                          b.emf_f[0], b.emf_f[1], b.Ecarry, b.Epre};
+         // the update writes nothing the constrained transport reads before
+         // KBfacesC2p (and reads no slopes, whose memory the edges take)
+         if (both)
+            DH_TRY(run_both(x, "update_edges_collect", ku, m.ntot, kc, m.ntot));
+         else
+            DH_TRY(run_ord(x, "edges_collect", kc, m.ntot, b.ord[ORD_CELLS]));
+         EdgeArgs ea{m, b.F[0], b.F[1], b.rng[0], b.rng[1], b.Epre, b.piph, b.dphi};
+         KEdgesFinal kef{ea, ct, b.wiph, b.emf_f[0], b.emf_f[1], b.Eo, b.Eown, b.Ecarry};
+         KUpdateB kb{m, RK, dt, b.F[0], b.F[1], b.rng[0], b.rng[1], b.Eo, st.pin, st.prk, st.pout};
+         KLineSteps<1> kl1{m, b.F[0], b.estep[0]};
+         KLineSteps<2> kl2{m, b.F[1], b.estep[1]};
+         KEdgeSegments ks{m, dt, b.F[0], b.F[1], b.estep[0], b.estep[1], b.lbase[0], b.lbase[1],
+                          b.piph, b.dphi, b.Eown, b.seg[0], b.seg[1]};
+         KEdgeAdjust ke{m, b.F[0], b.F[1], b.estep[0], b.estep[1], b.lbase[0], b.lbase[1],
+                        b.seg[0], b.seg[1], st.pout};
+         long nf = (long)b.F[0].n + b.F[1].n;
+         if (both && !reuse) {
+            KBoth<KLineSteps<1>, KLineSteps<2>> kl{kl1, kl2, b.F[0].n};
+            DH_TRY(run_both(x, "edges_final_line_steps", kef, m.ntot, kl, nf));
+         } else {
+            DH_TRY(run_ord(x, "edges_final", kef, m.ntot, b.ord[ORD_CELLS]));
+         }
+         if (both) {
+            DH_TRY(run_both(x, "update_B_edge_segments", kb, m.ntot, ks, nf));
+            DH_TRY(run_ord(x, "edge_adjust", ke, nf, b.ord[ORD_EDGES]));
+         } else {
+            DH_TRY(run_ord(x, "update_B", kb, m.ntot, b.ord[ORD_CELLS]));
+            if (dim_active(m, 2)) {
+               if (dim_active(m, 1) && !reuse)
+                  DH_TRY(run_ord(x, "line_steps_r", kl1, b.F[0].n, b.ord[ORD_FACES_R]));
+               if (!reuse)
+                  DH_TRY(run_ord(x, "line_steps_z", kl2, b.F[1].n, b.ord[ORD_FACES_Z]));
+               DH_TRY(run_ord(x, "edge_segments", ks, nf, b.ord[ORD_EDGES]));
+               DH_TRY(run_ord(x, "edge_adjust", ke, nf, b.ord[ORD_EDGES]));
+            }
+         }
+      }
+      if (!both || !mhd) DH_TRY(run_ord(x, "update", ku, m.ntot, b.ord[ORD_CELLS]));
+      if constexpr (mhd) {
+         if constexpr (HasFlipTracks<X>::value) {
+            if (first_step)
+               DH_TRY(x.flip_tracks(m, b.F[0], b.F[1], b.piph, b.wiph, dt, st.pout, st.pflip));
+         } else if (first_step) {
             for (int dim = 1; dim <= 2; ++dim) {
                int d = dim - 1;
                if (!dim_active(m, dim)) continue;
