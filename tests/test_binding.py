@@ -31,7 +31,7 @@ PLUG = os.path.join(REPO, "disco_amd", "plugins")
 sys.path.insert(0, os.path.join(HERE, "cpu_engine"))
 import build as cpu_build  # noqa: E402
 
-pytestmark = pytest.mark.skipif(not os.path.isdir(REF), reason="reference sources not mounted")
+pytestmark = pytest.mark.skipif(not os.path.isfile(f"{REF}/paul.h"), reason="reference sources not mounted")
 
 CORE = ["readpar.c", "timestep.c", "onestep.c", "riemann.c", "mpisetup.c", "gridsetup.c",
         "domain.c", "misc.c", "faces_alt.c", "exchange.c", "plm.c", "report.c", "profiler.c",
