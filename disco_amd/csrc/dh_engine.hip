@@ -162,12 +162,30 @@ struct KZeroWords {
    DHD void operator()(long i) const { p[i] = 0ull; }
 };
 
+// The quadrant of an angle x as the signs of its sine and cosine give it: 1
+// or 4, 0 for the others.  Away from the quadrants' edges the interval the
+// angle lies in decides; within 1e-6 of an edge, or outside [0, 2 pi], the
+// functions do.
+__device__ __forceinline__ int quadrant_1_or_4(double x)
+{
+   const double H = 0.5 * M_PI, E = 1e-6;
+   if (x > E && x < H - E) return 1;
+   if (x > 3.0 * H + E && x < 4.0 * H - E) return 4;
+   if (x > H + E && x < 3.0 * H - E) return 0;
+   double sn, cs;
+   sincos(x, &sn, &cs);
+   return sn > 0. && cs > 0. ? 1 : sn < 0. && cs > 0. ? 4 : 0;
+}
+
 // Start cell of every annulus (faces_alt.c:59-78): one wavefront per
-// annulus scans 64 cells at a time with ballots for the first cell in the
-// first quadrant that follows a cell in the fourth.
+// annulus scans 256 cells at a time, 64 by 64 with ballots, for the first
+// cell in the first quadrant that follows a cell in the fourth.  Its time
+// is the chain of batches: with 64 cells a batch and a sine and cosine for
+// every cell the 128-ring vortex took 8.2 us and 512 rings 38, now 7.4 and 32.
 // Block b of the launch (its TPB / 64 wavefronts take annuli 4 b .. 4 b + 3).
 __device__ __forceinline__ void ring_start_block(const Mesh &m, const double *piph, int *I0, unsigned blk)
 {
+   constexpr int U = 4;
    int a = blk * (TPB / 64) + threadIdx.x / 64;
    int lane = threadIdx.x & 63;
    if (a >= m.nann) return;
@@ -175,29 +193,28 @@ __device__ __forceinline__ void ring_start_block(const Mesh &m, const double *pi
    double convert = 2. * M_PI / m.Pmax;
    bool seen4 = false;
    int found = -1;
-   for (int base = 0; base < np; base += 64) {
-      int i = base + lane;
-      int quad = 0;
-      if (i < np) {
-         double sn, cs;
-         sincos(piph[c0 + i] * convert, &sn, &cs);
-         if (sn > 0. && cs > 0.) quad = 1;
-         else if (sn < 0. && cs > 0.) quad = 4;
+   for (int base = 0; base < np && found < 0; base += 64 * U) {
+      double x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         int i = base + 64 * u + lane;
+         x[u] = i < np ? piph[c0 + i] * convert : M_PI;  // (past the end: neither quadrant)
       }
-      unsigned long long b4 = __ballot(quad == 4);
-      unsigned long long b1 = __ballot(quad == 1);
-      unsigned long long cand = 0;
-      if (seen4) {
-         cand = b1;
-      } else if (b4) {
-         int f4 = __ffsll((long long)b4) - 1;
-         cand = f4 >= 63 ? 0ULL : (b1 & (~0ULL << (f4 + 1)));
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+         int quad = quadrant_1_or_4(x[u]);
+         unsigned long long b4 = __ballot(quad == 4);
+         unsigned long long b1 = __ballot(quad == 1);
+         unsigned long long cand = 0;
+         if (seen4) {
+            cand = b1;
+         } else if (b4) {
+            int f4 = __ffsll((long long)b4) - 1;
+            cand = f4 >= 63 ? 0ULL : (b1 & (~0ULL << (f4 + 1)));
+         }
+         if (cand && found < 0) found = base + 64 * u + __ffsll((long long)cand) - 1;
+         if (b4) seen4 = true;
       }
-      if (cand) {
-         found = base + __ffsll((long long)cand) - 1;
-         break;
-      }
-      if (b4) seen4 = true;
    }
    if (lane == 0) I0[a] = found < 0 ? 0 : found;
 }
@@ -508,19 +525,23 @@ __global__ __launch_bounds__(TPB) void k_report(Mesh m, dh_params P, DiagPlanet 
 
 // CFL reduction over real cells (misc.c:39-84).  Positive doubles order like
 // their bit patterns, so the minimum is an unsigned 64-bit atomic min, one
-// per workgroup; the grid is capped (MINDT_BLOCKS) and each thread takes
-// every stride-th cell, so that few atomics meet at the one address.
-constexpr unsigned MINDT_BLOCKS = 2048;
-// Block blk of nb blocks that share the cells (a grid-stride loop).
+// per workgroup; the grid is capped (MINDT_BLOCKS workgroups of MINDT_TPB)
+// and each thread takes every stride-th cell, so that few atomics meet at
+// the one address (with 2048 workgroups of 256 the two atomics of each cost
+// 20 us more than the sums).
+constexpr unsigned MINDT_BLOCKS = 512;
+constexpr int MINDT_TPB = 1024;
+// Block blk of nb blocks that share the cells (a grid-stride loop).  Thread
+// 0 returns once its minimum is in out.
 template <int NQ, class H>
 __device__ __forceinline__ void mindt_block(const Mesh &m, const dh_params &P, const double *prim,
                             const double *piph, const double *dphi, const double *wiph,
                             unsigned long long *out, unsigned blk, unsigned nb)
 {
-   __shared__ double red[TPB / 64];
-   long stride = (long)nb * TPB;
+   __shared__ double red[MINDT_TPB / 64];
+   long stride = (long)nb * blockDim.x;
    double dtc = HUGE_VAL;
-   for (long c = (long)blk * TPB + threadIdx.x; c < m.ntot; c += stride) {
+   for (long c = (long)blk * blockDim.x + threadIdx.x; c < m.ntot; c += stride) {
       double v = cell_mindt<NQ, H>(m, P, prim, piph, dphi, wiph, c);
       dtc = v < dtc ? v : dtc;
    }
@@ -533,16 +554,42 @@ __device__ __forceinline__ void mindt_block(const Mesh &m, const dh_params &P, c
    __syncthreads();
    if (threadIdx.x == 0) {
       double v = red[0];
-      for (int w = 1; w < TPB / 64; ++w) v = red[w] < v ? red[w] : v;
-      if (v < HUGE_VAL && v > 0.0) atomicMin(out, (unsigned long long)__double_as_longlong(v));
+      for (int w = 1; w < (int)blockDim.x / 64; ++w) v = red[w] < v ? red[w] : v;
+      if (v < HUGE_VAL && v > 0.0) {
+         unsigned long long old = atomicMin(out, (unsigned long long)__double_as_longlong(v));
+         asm volatile("" ::"v"(old) : "memory");  // (the use waits for the atomic)
+      }
    }
 }
+// A context's CFL reduction between calls: the minimum starts at +inf and
+// the count at 0, and the last workgroup to finish leaves them so.
+struct MinState {
+   unsigned long long min;
+   unsigned done;
+};
+constexpr unsigned long long MINDT_NONE = 0x7FF0000000000000ULL;  // +inf
+// The last workgroup stores the result in the host's pinned memory, where
+// the host reads it after the stream: a copy in of the start value and one
+// out of the result were two more launches around this one, of 3 to 5 us
+// each and their gaps, in every step.
 template <int NQ, class H>
-__global__ __launch_bounds__(TPB) void k_mindt(Mesh m, dh_params P, const double *prim,
+__global__ __launch_bounds__(MINDT_TPB) void k_mindt(Mesh m, dh_params P, const double *prim,
                                                const double *piph, const double *dphi,
-                                               const double *wiph, unsigned long long *out)
+                                               const double *wiph, MinState *st,
+                                               unsigned long long *host)
 {
-   mindt_block<NQ, H>(m, P, prim, piph, dphi, wiph, out, blockIdx.x, gridDim.x);
+   mindt_block<NQ, H>(m, P, prim, piph, dphi, wiph, &st->min, blockIdx.x, gridDim.x);
+   if (threadIdx.x == 0) {
+      // (no fence: both are device-scope atomics and this one is issued after
+      // the other has returned; a fence writes the whole L2 back, 55 us a
+      // call over the 2048 workgroups of a large mesh)
+      if (atomicAdd(&st->done, 1u) == gridDim.x - 1) {
+         unsigned long long v = atomicExch(&st->min, MINDT_NONE);
+         atomicExch(&st->done, 0u);
+         __atomic_store_n(host, v, __ATOMIC_RELAXED);
+         __threadfence_system();
+      }
+   }
 }
 
 // ---------------------------------------------------------------------------
@@ -721,7 +768,8 @@ struct HipExec {
    const void *gkey = nullptr;
    std::vector<TimerRow> rows;
    std::vector<void *> allocs;
-   unsigned long long *d_min = nullptr;
+   MinState *d_min = nullptr;
+   unsigned long long *h_min = nullptr;  // pinned
 
    // Brackets one launch with events when the timers are on.
    struct Bracket {
@@ -912,17 +960,15 @@ struct HipExec {
    int min_dt(const Mesh &m, const dh_params &P, const double *prim, const double *piph,
               const double *dphi, const double *wiph, double *out)
    {
-      unsigned long long init = 0x7FF0000000000000ULL;  // +inf
-      HIPCHK(hipMemcpyAsync(d_min, &init, sizeof init, hipMemcpyHostToDevice, stream));
       {
          Bracket b(*this, "mindt");
-         unsigned nb = nblocks(m.ntot) < MINDT_BLOCKS ? nblocks(m.ntot) : MINDT_BLOCKS;
-         k_mindt<NQ, H><<<nb, TPB, 0, stream>>>(m, P, prim, piph, dphi, wiph, d_min);
+         unsigned nb = (unsigned)((m.ntot + MINDT_TPB - 1) / MINDT_TPB);
+         if (nb > MINDT_BLOCKS) nb = MINDT_BLOCKS;
+         k_mindt<NQ, H><<<nb, MINDT_TPB, 0, stream>>>(m, P, prim, piph, dphi, wiph, d_min, h_min);
       }
       LAUNCH_CHECK();
-      unsigned long long bits = 0;
-      HIPCHK(hipMemcpyAsync(&bits, d_min, sizeof bits, hipMemcpyDeviceToHost, stream));
       HIPCHK(hipStreamSynchronize(stream));
+      unsigned long long bits = __atomic_load_n(h_min, __ATOMIC_RELAXED);
       memcpy(out, &bits, sizeof bits);
       return DH_OK;
    }
@@ -1098,6 +1144,7 @@ static void release(dh_ctx *c)
          (void)hipEventDestroy(pe.second);
       }
    for (void *p : c->x.allocs) (void)hipFree(p);
+   if (c->x.h_min) (void)hipHostFree(c->x.h_min);
    if (c->x.stream) (void)hipStreamDestroy(c->x.stream);
    delete c;
 }
@@ -1576,7 +1623,15 @@ int dh_create(const dh_grid *g, const dh_params *par, dh_ctx **out)
       delete c;
       return fail(DH_EHIP, "hipStreamCreate failed");
    }
-   int rc = c->x.alloc((void **)&c->x.d_min, sizeof(unsigned long long));
+   int rc = c->x.alloc((void **)&c->x.d_min, sizeof(MinState));
+   if (!rc) {
+      MinState init{MINDT_NONE, 0};
+      rc = c->x.put(c->x.d_min, &init, sizeof init);
+   }
+   if (!rc && hipHostMalloc((void **)&c->x.h_min, sizeof(unsigned long long)) != hipSuccess) {
+      c->x.h_min = nullptr;
+      rc = fail(DH_ENOMEM, "hipHostMalloc failed");
+   }
    if (!rc) rc = create_buffers(c->x, c->b, g, *par);
    if (!rc) rc = c->x.sync();
    if (rc) {
