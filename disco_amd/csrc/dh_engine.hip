@@ -232,31 +232,39 @@ __global__ __launch_bounds__(TPB) void k_ring_start(Mesh m, const double *piph, 
 // faces p + 1 and b - 1 share no cell: the batch's flagged faces fall into
 // runs, each run's first thread hands its run over in order, all runs at
 // once.  The result is the reference's face-by-face order: batches are in
-// order, and where a track of one batch closes on itself its last run waits
-// for the first unless those two share no cell either.  The flags are those
+// order, and where the track closes on itself around a batch its last run
+// waits for the first unless those two share no cell either.  The flags are those
 // of the owners before any flip: of the faces of a later batch only the
 // last one of the track can have changed owner (by a flip of face 0), so its
 // position is kept from the start.
 //
-// What bounds it: a chain of two loads and the longest run.  Flags in
-// launches of their own and one lane per track handing over its whole track
-// took 2 x (8 + 49) us a step on the 32 x 8 disk, whose shear flips most faces;
-// now 97.
+// What bounds it: the longest run, since where the shear moves the mesh by
+// a cell a step most faces flip.  So a batch with a flag holds its faces and
+// their cells' fluxes in LDS (by cell, so that two faces of one slot meet in
+// one word) and a run is a chain of LDS reads, not of memory latencies: one
+// lane per track and flips in memory took 2 x 49 us a step on the 32 x 8
+// disk and 2 x 111 on the 127 x 31 one, with 2 x 8 and 2 x 37 us more for
+// the flags in launches of their own; now 37 and 179 a step in all.
 template <int DIM>
 __device__ __forceinline__ void flip_track(const Mesh &m, const Faces &F, const double *piph,
                                            const double *wiph, double dt, double *Phi,
                                            double *rkPhi, int JK)
 {
+   constexpr int W = TPB + 2;        // a batch's faces (from 1 on) and the ones before and after
    __shared__ double s_up[TPB + 1];  // moved upper edges: [0] the face before the batch
    __shared__ unsigned long long s_flag[WAVES], s_start[WAVES];
+   __shared__ double s_P[2][W], s_rk[2][W];  // fluxes and their RK copies of the L and R cells
+   __shared__ short s_c[2][W];               // each face's L and R cell in those
+   __shared__ signed char s_LR[W];
    if (track_skipped(F.npairs, JK)) return;
    const int base = F.fI[JK], N = F.fI[JK + 1] - base;
    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+   const size_t nt = (size_t)m.ntot;
+   double *const Phis[2] = {Phi + (DIM == 1 ? 2 : 4) * nt, Phi + (DIM == 1 ? 1 : 3) * nt};
+   double *const rks[2] = {rkPhi + (DIM == 1 ? 2 : 4) * nt, rkPhi + (DIM == 1 ? 1 : 3) * nt};
+   const Pair pr = pair_of(m, DIM, JK);
+   const int np[2] = {m.Np[pr.a], m.Np[pr.b]};
    KFlipFlags<DIM> k{m, F, piph, wiph, &dt, nullptr};
-   // whether faces f and g of the track (0 <= f, g < N) share a cell
-   auto share = [&](int f, int g) {
-      return F.L[base + f] == F.L[base + g] || F.R[base + f] == F.R[base + g];
-   };
    // the next bit at or after i, and the last one before i (-1: none)
    auto next_bit = [&](const unsigned long long *b, int i) {
       for (int w = i >> 6; w < WAVES; ++w) {
@@ -275,8 +283,9 @@ __device__ __forceinline__ void flip_track(const Mesh &m, const Faces &F, const 
       return -1;
    };
    const double last = k.moved_up(base + N - 1);
+   const bool one = N <= TPB;  // the whole track in one batch
    for (int n0 = 0; n0 < N; n0 += TPB) {
-      const int n = n0 + tid;
+      const int n = n0 + tid, cnt = N - n0 < TPB ? N - n0 : TPB;
       double up = 0.0;
       if (n < N) up = n == N - 1 ? last : k.moved_up(base + n);
       double prev = n0 == 0 ? last : s_up[TPB];  // (the last batch's final edge)
@@ -288,27 +297,76 @@ __device__ __forceinline__ void flip_track(const Mesh &m, const Faces &F, const 
       unsigned long long b = __ballot(flag);
       if (lane == 0) s_flag[wv] = b;
       if (!__syncthreads_or(flag)) continue;
+      // the batch's faces, with the ones on either side where those are not
+      // in it (one face where the track is one longer than the batch), and
+      // their cells counted from the first of these faces'
+      const bool meet = N == cnt + 1;
+      const int w0 = one ? 1 : 0, w1 = one || meet ? cnt : cnt + 1;
+      const int fr = base + (one ? 0 : (n0 + N - 1) % N);
+      for (int i = w0 + tid; i <= w1; i += TPB) {
+         int f = base + (n0 + i - 1 + N) % N;
+         s_LR[i] = F.LR[f];
+#pragma unroll
+         for (int h = 0; h < 2; ++h) {
+            int c = h == 0 ? F.L[f] : F.R[f], c0 = h == 0 ? F.L[fr] : F.R[fr];
+            int r = c - c0;
+            if (r < 0) r += np[h];
+            if (r >= W) r = 0;  // (only where non-finite positions left no face list)
+            s_c[h][i] = (short)r;
+            s_P[h][r] = Phis[h][c];
+            s_rk[h][r] = rks[h][c];
+         }
+      }
+      __syncthreads();
+      // whether faces i and j of the batch share a cell
+      auto share = [&](int i, int j) { return s_c[0][i] == s_c[0][j] || s_c[1][i] == s_c[1][j]; };
+      auto before = [&](int i) { return i > 1 || !one ? i - 1 : cnt; };
+      auto after = [&](int i) { return i < cnt ? i + 1 : one ? 1 : meet ? 0 : cnt + 1; };
       bool start = false;
       if (flag) {
          int p = last_bit(s_flag, tid);
-         start = p < 0 || (tid - p > 2 && !share(n0 + p + 1, n - 1));
+         start = p < 0 || (tid - p > 2 && !share(p + 2, tid));  // (faces p + 1 and tid - 1)
       }
       b = __ballot(start);
       if (lane == 0) s_start[wv] = b;
       __syncthreads();
       int end = start ? next_bit(s_start, tid + 1) : tid;
       bool wait = false;
-      if (start && N <= TPB && end == TPB) {  // the last run of a one-batch track
+      if (start && end == TPB) {  // the last run: its far side may meet the first's
          int l = next_bit(s_flag, 0), h = last_bit(s_flag, TPB);
          if (next_bit(s_start, 0) != tid)  // (a single run has nothing to wait for)
-            wait = l + N - h <= 2 || share((h + 1) % N, (l + N - 1) % N);
+            wait = l + N - h <= 2 || share(after(h + 1), before(l + 1));
       }
       for (int phase = 0; phase < 2; ++phase) {
          if (start && wait == (phase == 1))
-            for (int i = tid; i < end; i = next_bit(s_flag, i + 1))
-               flip_one(DIM, (size_t)m.ntot, F, base, N, n0 + i, Phi, rkPhi);
+            for (int i = tid; i < end; i = next_bit(s_flag, i + 1)) {
+               // flip_one on the batch's copies
+               int f = i + 1, fm = before(f), fp = after(f);
+               int hf = s_LR[f] != 0, hm = s_LR[fm] != 0, hp = s_LR[fp] != 0;
+               int P = s_c[hf][f], Pm = s_c[hm][fm], Pp = s_c[hp][fp];
+               double ph = s_P[hf][P], rk = s_rk[hf][P];
+               s_P[hf][P] = s_P[hm][Pm] + ph;
+               s_rk[hf][P] = s_rk[hm][Pm] + rk;
+               s_P[hm][Pm] = -ph;
+               s_rk[hm][Pm] = -rk;
+               s_P[hp][Pp] = s_P[hp][Pp] + ph;
+               s_rk[hp][Pp] = s_rk[hp][Pp] + rk;
+               s_LR[f] = (signed char)!s_LR[f];
+               s_LR[fm] = (signed char)!s_LR[fm];
+            }
          __syncthreads();
       }
+      for (int i = w0 + tid; i <= w1; i += TPB) {
+         int f = base + (n0 + i - 1 + N) % N;
+         F.LR[f] = s_LR[i];
+#pragma unroll
+         for (int h = 0; h < 2; ++h) {
+            int c = h == 0 ? F.L[f] : F.R[f];
+            Phis[h][c] = s_P[h][s_c[h][i]];
+            rks[h][c] = s_rk[h][s_c[h][i]];
+         }
+      }
+      __syncthreads();
    }
 }
 // The tracks of both directions (they share no flux slot): the r tracks,

@@ -56,3 +56,35 @@ def test_long_annuli_step_as_the_host_build(cname, over):
     print("  worst", compare_states(gpu.download(a), cpu.download(a)), flush=True)
     gpu.close()
     cpu.close()
+
+
+@pytest.mark.parametrize("aspect", [0.5, 0.12, 0.06, 0.03])
+def test_flips_of_strong_shear(aspect):
+    """Keplerian shear of about a cell a step flips most faces: tracks of
+    fewer faces than a flip batch (256), about as many, and several batches,
+    with runs that cross batches and the track's closure.  Steps from common
+    states: a trajectory of this mesh is ill-conditioned (the host build's
+    own moves by 1e-10 under a one-ulp change of libm)."""
+    import sys
+    sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpu_engine"))
+    import build as cpu_build
+    from helpers import compare_states
+    cfg, par, a = _initial("mhd_kep", {"Num_R": 6, "Num_Z": 3, "aspect": aspect})
+    print(f"case flips aspect {aspect}: annuli of {a.np_.min()} to {a.np_.max()} cells", flush=True)
+    lib = capi.load_library(cpu_build.build())
+    lib.dhx_flip_count.argtypes = [__import__("ctypes").c_void_p]
+    lib.dhx_flip_count.restype = __import__("ctypes").c_long
+    cpu = capi.DiscoHip(cfg, par, a, library=lib)
+    s = a
+    for n in range(4):
+        gpu = capi.DiscoHip(cfg, par, s)
+        # at most about a cell of shear between neighbouring annuli
+        dt = min(cpu.getmindt(), 2 * np.pi / s.np_.max())
+        gpu.timestep(dt)
+        cpu.timestep(dt)
+        s = cpu.download(s)
+        print(f"  step {n}: {lib.dhx_flip_count(cpu.ctx)} flips so far, worst",
+              compare_states(gpu.download(s), s, tol=1e-9), flush=True)
+        gpu.close()
+    assert lib.dhx_flip_count(cpu.ctx) > a.n_real() // 10
+    cpu.close()
