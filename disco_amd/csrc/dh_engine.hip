@@ -92,6 +92,20 @@ template <class K1, class K2>
 struct ByElements<KBoth<K1, K2>> {
    static constexpr bool value = ByElements<K1>::value || ByElements<K2>::value;
 };
+// Whether a kernel runs by tiles always (its lanes take values from each
+// other).
+template <class K, class = void>
+struct ByTilesOnly {
+   static constexpr bool value = false;
+};
+template <class K>
+struct ByTilesOnly<K, decltype((void)K::by_tiles_only)> {
+   static constexpr bool value = true;
+};
+template <class K1, class K2>
+struct ByTilesOnly<KBoth<K1, K2>> {
+   static constexpr bool value = ByTilesOnly<K1>::value || ByTilesOnly<K2>::value;
+};
 // Whether the tiles are worth their idle lanes: at least 0.94 of the lanes
 // at work (annuli of 500 cells and more).  At 0.95 (the 127 x 31 disk) a
 // step gains 4%, at 0.92 (the 128-ring vortex) it loses 4%, at 0.8 (the
@@ -117,6 +131,32 @@ __device__ __forceinline__ void tile_wave(const K &k, const TileList &tl, int w,
    t.group = __builtin_amdgcn_readfirstlane(t.group);
    t.dim = __builtin_amdgcn_readfirstlane(t.dim);
    if (lane < t.n) k.at(t.first + lane, t.group, t.dim);
+}
+__device__ __forceinline__ void tile_wave(const KEdgesCollectAvg &k, const TileList &tl, int w,
+                                          int lane)
+{
+   if (w >= tl.n) return;
+   Tile t = tl.t[w];
+   t.first = __builtin_amdgcn_readfirstlane(t.first);
+   t.n = __builtin_amdgcn_readfirstlane(t.n);
+   const int a = __builtin_amdgcn_readfirstlane(t.group);
+   const Mesh &m = k.k.m;
+   const size_t nt = (size_t)m.ntot;
+   long c = t.first + lane;
+   if (c >= m.off[a] + m.Np[a]) c -= m.Np[a];  // (the last tile's neighbour is the ring's first)
+   double E[8], B[8];
+#pragma unroll
+   for (int s = 0; s < 8; ++s) E[s] = B[s] = 0.0;
+   if (lane <= t.n) k.k.sums(c, a, E, B);
+#pragma unroll
+   for (int i = 0; i < 4; ++i) {
+      const int s = i < 2 ? i : i + 2;  // slots 0, 1, 4, 5
+      double e = __shfl_down(E[s + 2], 1, 64), b = __shfl_down(B[s + 2], 1, 64);
+      if (lane < t.n) {
+         k.k.Epre[i * nt + c] = .5 * (E[s] + e);
+         k.k.Epre[(4 + i) * nt + c] = .5 * (B[s] + b);
+      }
+   }
 }
 template <class K1, class K2>
 __device__ __forceinline__ void tile_wave(const KBoth<K1, K2> &k, const TileList &, int w, int lane)
@@ -888,7 +928,12 @@ struct HipExec {
    {
       if (n <= 0) return DH_OK;
       bool tiled = false;
-      if constexpr (!ByElements<K>::value) tiled = by_tiles(tiles_of(k), n);
+      if constexpr (ByTilesOnly<K>::value) {
+         tiled = true;
+         nord = 0;  // (its tiles are in storage order only)
+      } else if constexpr (!ByElements<K>::value) {
+         tiled = by_tiles(tiles_of(k), n);
+      }
       int row = (int)(&tune_row(name, 2 + (tiled ? nord : 0), strips, XcdContiguous<K>::value ? 1 : 0) -
                       tunes.data());
       TuneRow &t = tunes[row];
@@ -909,7 +954,9 @@ struct HipExec {
                long nt = (long)tl.n * 64;
                k_tiles<K><<<v == 0 ? nblocks(nt) : nblocks_xcd(nt), TPB, 0, stream>>>(k, tl, v != 0);
             }
-         if (!tiled) k_elems<K><<<v == 0 ? nblocks(n) : nblocks_xcd(n), TPB, 0, stream>>>(k, n, v);
+         if constexpr (!ByTilesOnly<K>::value)
+            if (!tiled)
+               k_elems<K><<<v == 0 ? nblocks(n) : nblocks_xcd(n), TPB, 0, stream>>>(k, n, v);
       }
       LAUNCH_CHECK();
       if (timing) {
@@ -1180,6 +1227,7 @@ struct HipExec {
       return DH_OK;
    }
    static constexpr bool merges_launches() { return true; }
+   static constexpr bool edge_means = true;
 };
 
 struct dh_ctx {
@@ -1470,6 +1518,7 @@ struct GroupExec {
    }
    // Every member must record the same launch sequence.
    static constexpr bool merges_launches() { return false; }
+   static constexpr bool edge_means = true;
 };
 
 // One launch of an ensemble: the ops of every mesh in device memory and

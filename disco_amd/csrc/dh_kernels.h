@@ -1109,10 +1109,21 @@ struct KEdgesCollect {
    DHD void at(long c, int a, int) const
    {
       size_t nt = (size_t)m.ntot;
+      double E[8], B[8];
+      sums(c, a, E, B);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+         Epre[s * nt + c] = E[s];
+         Epre[(8 + s) * nt + c] = B[s];
+      }
+   }
+   // The edges of cell c.
+   DHD void sums(long c, int a, double *E, double *B) const
+   {
+      size_t nt = (size_t)m.ntot;
       int c0 = m.off[a], np = m.Np[a];
       long cm = c == c0 ? c0 + np - 1 : c - 1;
       int j = a % m.Nr, k = a / m.Nr;
-      double E[8], B[8];
       if (phi_in_range(m, ct, j, k)) {
          double Ez = emf_phi[0 * nt + c], Br = emf_phi[1 * nt + c];
          double Er = emf_phi[2 * nt + c], Bz = emf_phi[3 * nt + c];
@@ -1134,6 +1145,7 @@ struct KEdgesCollect {
          }
       }
       double dpc = dphi[c];
+#pragma unroll
       for (int dim = 1; dim <= 2; ++dim) {
          if (!dim_active(m, dim)) continue;
          const Faces &F = dim == 1 ? Fr : Fz;
@@ -1166,23 +1178,37 @@ struct KEdgesCollect {
             acc(cr.base_out, cr.out_t0, cr.out_t1, o0);
          }
       }
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-         Epre[s * nt + c] = E[s];
-         Epre[(8 + s) * nt + c] = B[s];
-      }
    }
+};
+
+// The same with the mean of each phi edge over the two cells that hold it
+// (avg_Efields, first part) formed at once: the lanes of a wavefront take
+// consecutive cells of a ring, the upper neighbour's edges come from the
+// next lane, and of the lanes' cells (n + 1 of them, by m.atiles of at most
+// 63) all but the last are stored.  So 8 numbers a cell are written and read
+// again instead of 16, and a later gather reads one where it read two.
+// 127 x 31 MHD disk: 179 -> 171 us here, 266 -> 191 in KEdgesFinal.
+struct KEdgesCollectAvg {
+   KEdgesCollect k;
+   static constexpr bool by_tiles_only = true;
+   DHD TileList tiles() const { return k.m.atiles; }
 };
 
 // avg_Efields, first part (bfields.c:400-441), evaluated where it is read:
 // each phi-edge takes the mean of the values its two cells hold.  Slot s of
-// E (h = 0) or B (h = 1) of cell c of annulus a.
+// E (h = 0) or B (h = 1) of cell c of annulus a.  With AVG, Epre holds the
+// means (KEdgesCollectAvg): of slots {0, 1, 4, 5} of E, then of B.
+template <bool AVG>
 DHD double edge_avg(const Mesh &m, const double *Epre, int h, int s, long c, int a)
 {
    size_t nt = (size_t)m.ntot;
    const double *X = Epre + (size_t)h * 8 * nt;
    int c0 = m.off[a], np = m.Np[a];
    int e = s & 3, base = s & 4;
+   if (AVG) {
+      long o = e < 2 ? c : c == c0 ? c0 + np - 1 : c - 1;
+      return Epre[(size_t)(4 * h + base / 2 + (e & 1)) * nt + o];
+   }
    if (e < 2) {
       long cp = c - c0 == np - 1 ? c0 : c + 1;
       return .5 * (X[(base + e) * nt + c] + X[(base + e + 2) * nt + cp]);
@@ -1196,6 +1222,7 @@ DHD double edge_avg(const Mesh &m, const double *Epre, int h, int s, long c, int
 // cell's two corner values interpolated in phi; E in *fE, B in *fB.  Each
 // face's edge is read by one cell, the face's owner (edges_post_face), which
 // forms it where it reads it.  The face's cells are of annuli aL and aR.
+template <bool AVG>
 DHD void face_emf(const Mesh &m, int dim, int aL, int aR, const Faces &F, const double *piph,
                   const double *dphi, const double *Epre, int f, double *fE, double *fB)
 {
@@ -1208,10 +1235,10 @@ DHD void face_emf(const Mesh &m, int dim, int aL, int aR, const Faces &F, const 
    int eL = dim == 1 ? 1 : 5, eR = dim == 1 ? 0 : 4;
    // LRtype 0: the face ends at L's upper edge; R's corners are interpolated
    int eo = LR == 0 ? eL : eR, ec = LR == 0 ? eR : eL;
-   double Ea = (dp2 * edge_avg(m, Epre, 0, ec, c2, a2) + dp1 * edge_avg(m, Epre, 0, ec + 2, c2, a2)) / (dp1 + dp2);
-   double Ba = (dp2 * edge_avg(m, Epre, 1, ec, c2, a2) + dp1 * edge_avg(m, Epre, 1, ec + 2, c2, a2)) / (dp1 + dp2);
-   *fE = .5 * (edge_avg(m, Epre, 0, eo, c1, a1) + Ea);
-   *fB = .5 * (edge_avg(m, Epre, 1, eo, c1, a1) + Ba);
+   double Ea = (dp2 * edge_avg<AVG>(m, Epre, 0, ec, c2, a2) + dp1 * edge_avg<AVG>(m, Epre, 0, ec + 2, c2, a2)) / (dp1 + dp2);
+   double Ba = (dp2 * edge_avg<AVG>(m, Epre, 1, ec, c2, a2) + dp1 * edge_avg<AVG>(m, Epre, 1, ec + 2, c2, a2)) / (dp1 + dp2);
+   *fE = .5 * (edge_avg<AVG>(m, Epre, 0, eo, c1, a1) + Ea);
+   *fB = .5 * (edge_avg<AVG>(m, Epre, 1, eo, c1, a1) + Ba);
 }
 
 // The four phi+ edges of a cell after avg_Efields, before the advective
@@ -1224,28 +1251,29 @@ struct EdgeArgs {
    const double *Epre, *piph, *dphi;
 };
 
+template <bool AVG>
 DHD void edges_post_face(const EdgeArgs &g, long c, int a, double *out)
 {
    const Mesh &m = g.m;
    const int slots[4] = {0, 1, 4, 5};
 #pragma unroll
    for (int s = 0; s < 4; ++s) {
-      out[s] = edge_avg(m, g.Epre, 0, slots[s], c, a);
-      out[4 + s] = edge_avg(m, g.Epre, 1, slots[s], c, a);
+      out[s] = edge_avg<AVG>(m, g.Epre, 0, slots[s], c, a);
+      out[4 + s] = edge_avg<AVG>(m, g.Epre, 1, slots[s], c, a);
    }
    if (m.Nr > 1) {
       CellRanges cr = load_ranges(m, 1, g.rngr, g.Fr.fI, c, a);
       if (cr.in)
-         face_emf(m, 1, a - 1, a, g.Fr, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[0], &out[4]);
+         face_emf<AVG>(m, 1, a - 1, a, g.Fr, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[0], &out[4]);
       if (cr.out)
-         face_emf(m, 1, a, a + 1, g.Fr, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[1], &out[5]);
+         face_emf<AVG>(m, 1, a, a + 1, g.Fr, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[1], &out[5]);
    }
    if (m.Nz > 1) {
       CellRanges cr = load_ranges(m, 2, g.rngz, g.Fz.fI, c, a);
       if (cr.in)
-         face_emf(m, 2, a - m.Nr, a, g.Fz, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[2], &out[6]);
+         face_emf<AVG>(m, 2, a - m.Nr, a, g.Fz, g.piph, g.dphi, g.Epre, cr.base_in + cr.in_h1, &out[2], &out[6]);
       if (cr.out)
-         face_emf(m, 2, a, a + m.Nr, g.Fz, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[3], &out[7]);
+         face_emf<AVG>(m, 2, a, a + m.Nr, g.Fz, g.piph, g.dphi, g.Epre, cr.base_out + cr.out_h1, &out[3], &out[7]);
    }
 }
 
@@ -1253,6 +1281,7 @@ DHD void edges_post_face(const EdgeArgs &g, long c, int a, double *out)
 // (subtract_advective_B_fluxes, bfields.c:646-690): Eo = {E0, E1, E4, E5}.
 // Also E_phi of each owned face, Eown = {r-in, r-out, z-in, z-out}, and the
 // full edge state of cells outside the phi-flux range (Ecarry).
+template <bool AVG>
 struct KEdgesFinal {
    EdgeArgs g;
    int ct;
@@ -1266,7 +1295,7 @@ struct KEdgesFinal {
       size_t nt = (size_t)m.ntot;
       int j = a % m.Nr, k = a / m.Nr;
       double v[8];
-      edges_post_face(g, c, a, v);
+      edges_post_face<AVG>(g, c, a, v);
       double own[4] = {0.0, 0.0, 0.0, 0.0};
       if (m.Nr > 1) {
          size_t nfs = (size_t)g.Fr.n;
@@ -1300,7 +1329,7 @@ struct KEdgesFinal {
          int c0 = m.off[a], np = m.Np[a];
          long cm = c == c0 ? c0 + np - 1 : c - 1;
          double vm[8];
-         edges_post_face(g, cm, a, vm);
+         edges_post_face<AVG>(g, cm, a, vm);
          double Ec[8] = {E0, E1, vm[0], vm[1], E4, E5, vm[2], vm[3]};
          double Bc[8] = {v[4], v[5], vm[4], vm[5], v[6], v[7], vm[6], vm[7]};
 #pragma unroll

@@ -44,6 +44,7 @@ struct Mesh {
    const int *I0;        // [nann] ring start cells of the current substep
    TileList tiles;       // the cells in storage order
    TileList etiles;      // the faces of both directions (r, then z) in storage order
+   TileList atiles;      // the cells again, 63 a tile
 };
 
 // One ring of cells read from its start cell I0: element x (0 <= x <= N) is

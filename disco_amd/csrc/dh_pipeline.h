@@ -238,12 +238,12 @@ struct GroupSeq {
 };
 
 template <class X>
-int put_tiles(X &x, TileList &out, const GroupSeq &s)
+int put_tiles(X &x, TileList &out, const GroupSeq &s, int most = TILE)
 {
    std::vector<Tile> t;
    for (size_t p = 0; p < s.first.size(); ++p)
-      for (int i = 0; i < s.size[p]; i += TILE)
-         t.push_back({s.first[p] + i, s.size[p] - i < TILE ? s.size[p] - i : TILE, s.group[p],
+      for (int i = 0; i < s.size[p]; i += most)
+         t.push_back({s.first[p] + i, s.size[p] - i < most ? s.size[p] - i : most, s.group[p],
                       s.dim[p]});
    Tile *d = nullptr;
    DH_TRY(alloc_n(x, &d, sizeof(Tile) * (t.empty() ? 1 : t.size())));
@@ -314,6 +314,7 @@ int build_orders(X &x, Buffers &b, const std::vector<int> *fI)
       GroupSeq seq[ORD_KINDS], edges;
       sequences(order, seq);
       DH_TRY(put_tiles(x, m.tiles, seq[ORD_CELLS]));
+      if (b.mhd) DH_TRY(put_tiles(x, m.atiles, seq[ORD_CELLS], TILE - 1));
       for (int d = 0; d < 2; ++d) {
          const GroupSeq &f = seq[ORD_FACES_R + d];
          DH_TRY(put_tiles(x, b.F[d].tiles, f));
@@ -377,6 +378,17 @@ struct HasGhostRings {
 template <class X>
 struct HasGhostRings<X, decltype((void)&X::template ghost_rings<5>)> {
    static constexpr bool value = true;
+};
+
+// Whether an executor's lanes can form the phi edges' means as the edges are
+// collected (KEdgesCollectAvg).
+template <class X, class = void>
+struct HasEdgeMeans {
+   static constexpr bool value = false;
+};
+template <class X>
+struct HasEdgeMeans<X, decltype((void)X::edge_means)> {
+   static constexpr bool value = X::edge_means;
 };
 
 // Allocates and fills every buffer of a validated mesh.
@@ -746,8 +758,16 @@ struct Engine {
                         b.rng[0], b.rng[1], b.F[0].n, b.F[1].n};
       if constexpr (mhd) {
          int ct = P.ct;
-         KEdgesCollect kc{m, ct, b.dphi, b.emf_phi, b.F[0], b.F[1], b.rng[0], b.rng[1],
-                          b.emf_f[0], b.emf_f[1], b.Ecarry, b.Epre};
+         // (not for grmhd2: the compiler rounds the means' sums otherwise in
+         // this form, by an ulp, and the relativistic HLLD disk's branches
+         // turn an ulp into 1e-2 within a few steps)
+         constexpr bool avg = HasEdgeMeans<X>::value && !IsGR<H>::value;
+         KEdgesCollect kcells{m, ct, b.dphi, b.emf_phi, b.F[0], b.F[1], b.rng[0], b.rng[1],
+                              b.emf_f[0], b.emf_f[1], b.Ecarry, b.Epre};
+         auto kc = [&] {
+            if constexpr (avg) return KEdgesCollectAvg{kcells};
+            else return kcells;
+         }();
          // the update writes nothing the constrained transport reads before
          // KBfacesC2p (and reads no slopes, whose memory the edges take)
          if (both)
@@ -755,7 +775,7 @@ struct Engine {
          else
             DH_TRY(run_ord(x, "edges_collect", kc, m.ntot, b.ord[ORD_CELLS]));
          EdgeArgs ea{m, b.F[0], b.F[1], b.rng[0], b.rng[1], b.Epre, b.piph, b.dphi};
-         KEdgesFinal kef{ea, ct, b.wiph, b.emf_f[0], b.emf_f[1], b.Eo, b.Eown, b.Ecarry};
+         KEdgesFinal<avg> kef{ea, ct, b.wiph, b.emf_f[0], b.emf_f[1], b.Eo, b.Eown, b.Ecarry};
          KUpdateB kb{m, RK, dt, b.F[0], b.F[1], b.rng[0], b.rng[1], b.Eo, st.pin, st.prk, st.pout};
          KLineSteps<1> kl1{m, b.F[0], b.estep[0]};
          KLineSteps<2> kl2{m, b.F[1], b.estep[1]};

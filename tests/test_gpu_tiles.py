@@ -88,3 +88,30 @@ def test_flips_of_strong_shear(aspect):
         gpu.close()
     assert lib.dhx_flip_count(cpu.ctx) > a.n_real() // 10
     cpu.close()
+
+
+@pytest.mark.parametrize("cells", [5, 62, 63, 64, 65, 126, 127])
+def test_edge_means_at_the_tiles_ends(cells):
+    """The phi edges' means are formed by tiles of 63 cells, the last cell's
+    from the next tile's first or the ring's: annuli of one short tile, of
+    whole ones, and of one cell more and less."""
+    import sys
+    sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpu_engine"))
+    import build as cpu_build
+    from helpers import compare_states
+    # Np = floor(2 pi r / (aspect dr)), r the ring's outer radius: of eight
+    # rings from 0.5 to 2 (whose ghost rings stay at r > 0) the innermost
+    dr = 1.5 / 8
+    aspect = 2 * np.pi * (0.5 + dr) / (dr * (cells + 0.5))
+    cfg, par, a = _initial("mhd_kep", {"Num_R": 8, "Num_Z": 2, "aspect": aspect})
+    print(f"case edge means: annuli of {sorted(set(a.np_.tolist()))} cells", flush=True)
+    assert cells in a.np_
+    gpu = capi.DiscoHip(cfg, par, a)
+    cpu = capi.DiscoHip(cfg, par, a, library=capi.load_library(cpu_build.build()))
+    for _ in range(3):
+        dt = min(gpu.getmindt(), 1e-4)
+        gpu.timestep(dt)
+        cpu.timestep(dt)
+    print("  worst", compare_states(gpu.download(a), cpu.download(a)), flush=True)
+    gpu.close()
+    cpu.close()
