@@ -263,6 +263,20 @@ __global__ __launch_bounds__(TPB) void k_ring_start(Mesh m, const double *piph, 
    ring_start_block(m, piph, I0, blockIdx.x);
 }
 
+// A kernel by elements in the first nb workgroups and the ring starts in the
+// rest.
+template <class K>
+__global__ __launch_bounds__(TPB) void k_elems_rings(K k, long n, unsigned nb, Mesh m,
+                                                     const double *piph, int *I0)
+{
+   if (blockIdx.x < nb) {
+      long t = (long)blockIdx.x * TPB + threadIdx.x;
+      if (t < n) k(t);
+   } else {
+      ring_start_block(m, piph, I0, blockIdx.x - nb);
+   }
+}
+
 // check_flipped and flip_fluxes (bfields.c:693-814): one workgroup per face
 // track takes TPB faces at a time, each thread the flag of one face, and
 // hands the flagged faces over.  A flip of face n reads and writes fluxes of
@@ -996,6 +1010,21 @@ struct HipExec {
       {
          Bracket b(*this, "ring_start");
          k_ring_start<<<(unsigned)((m.nann + 3) / 4), TPB, 0, stream>>>(m, piph, I0);
+      }
+      LAUNCH_CHECK();
+      return DH_OK;
+   }
+
+   static constexpr bool rings_beside = true;
+   template <class K>
+   int run_beside_rings(const char *name, const K &k, long n, const Mesh &m, const double *piph,
+                        int *I0)
+   {
+      unsigned nb = nblocks(n);
+      {
+         Bracket b(*this, name);
+         k_elems_rings<K><<<nb + (unsigned)((m.nann + 3) / 4), TPB, 0, stream>>>(k, n, nb, m, piph,
+                                                                               I0);
       }
       LAUNCH_CHECK();
       return DH_OK;

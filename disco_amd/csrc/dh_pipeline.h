@@ -380,6 +380,17 @@ struct HasGhostRings<X, decltype((void)&X::template ghost_rings<5>)> {
    static constexpr bool value = true;
 };
 
+// Whether an executor can find the ring starts in the launch of another
+// kernel (run_beside_rings).
+template <class X, class = void>
+struct HasRingsBeside {
+   static constexpr bool value = false;
+};
+template <class X>
+struct HasRingsBeside<X, decltype((void)X::rings_beside)> {
+   static constexpr bool value = X::rings_beside;
+};
+
 // Whether an executor's lanes can form the phi edges' means as the edges are
 // collected (KEdgesCollectAvg).
 template <class X, class = void>
@@ -587,19 +598,23 @@ struct Engine {
    // slopes when grads is set (plm.c:56-232).  With reuse the buffers
    // already hold the faces of the current positions and only the slopes
    // are formed.
+   // rings: the ring starts are those of the current positions already.
    template <int NQ>
-   int topology(bool grads, bool reuse = false)
+   int topology(bool grads, bool reuse = false, bool rings = false)
    {
       const Mesh &m = b.m;
       if (!dim_active(m, 1) && !dim_active(m, 2)) return DH_OK;
-      if (!reuse) DH_TRY(x.ring_start(m, b.piph, b.I0));
+      if (!reuse && !rings) DH_TRY(x.ring_start(m, b.piph, b.I0));
       if (merged() && dim_active(m, 1) && dim_active(m, 2)) return topology_merged<NQ>(grads, reuse);
       for (int dim = 1; dim <= 2; ++dim) {
          int d = dim - 1;
          if (!dim_active(m, dim)) continue;
          double *grad = dim == 1 ? b.gradr : b.gradz;
          bool slopes = grads && b.P.plm != 0.0;
-         if (!reuse && dim == 1) {
+         if (!reuse && dim == 1 && merged()) {
+            KRangesFaces<1> f1{{m, b.piph, b.rng[d]}, {m, b.F[d], b.rng[d], b.piph, b.dphi}};
+            DH_TRY(run_ord(x, "faces_r", f1, m.ntot, b.ord[ORD_CELLS]));
+         } else if (!reuse && dim == 1) {
             DH_TRY(run_ord(x, "ranges_r", KCellRanges<1>{m, b.piph, b.rng[d]}, m.ntot, b.ord[ORD_CELLS]));
             DH_TRY(run_ord(x, "faces_r", KFaces<1>{m, b.F[d], b.rng[d], b.piph, b.dphi}, m.ntot,
                            b.ord[ORD_CELLS]));
@@ -638,11 +653,8 @@ struct Engine {
    {
       const Mesh &m = b.m;
       if (!reuse) {
-         KCellRanges<1> r1{m, b.piph, b.rng[0]};
-         KCellRanges<2> r2{m, b.piph, b.rng[1]};
-         DH_TRY(run_both(x, "ranges", r1, m.ntot, r2, m.ntot));
-         KFaces<1> f1{m, b.F[0], b.rng[0], b.piph, b.dphi};
-         KFaces<2> f2{m, b.F[1], b.rng[1], b.piph, b.dphi};
+         KRangesFaces<1> f1{{m, b.piph, b.rng[0]}, {m, b.F[0], b.rng[0], b.piph, b.dphi}};
+         KRangesFaces<2> f2{{m, b.piph, b.rng[1]}, {m, b.F[1], b.rng[1], b.piph, b.dphi}};
          DH_TRY(run_both(x, "faces", f1, m.ntot, f2, m.ntot));
       }
       if (!grads) return DH_OK;
@@ -725,7 +737,21 @@ struct Engine {
       const bool both = merge && dim_active(m, 1) && dim_active(m, 2);
       KWcell<NQ, H> kw{m, P, b.prim, b.wiph};
       KPlmPhi<NQ> kpl{m, P.plm, b.prim, b.dphi, b.gradp};
-      if (first_step && merge && P.mesh_motion != 3) {
+      // on small meshes the ring starts (of the same positions) go with them
+      bool rings = false;
+      if constexpr (HasRingsBeside<X>::value)
+         rings = merge && !reuse && (dim_active(m, 1) || dim_active(m, 2)) &&
+                 !(first_step && P.mesh_motion == 3);
+      if (rings) {
+         if constexpr (HasRingsBeside<X>::value) {
+            if (first_step)
+               DH_TRY(x.run_beside_rings("wcell_plm_phi_rings",
+                                         KBoth<KWcell<NQ, H>, KPlmPhi<NQ>>{kw, kpl, m.ntot},
+                                         2L * m.ntot, m, b.piph, b.I0));
+            else
+               DH_TRY(x.run_beside_rings("plm_phi_rings", kpl, m.ntot, m, b.piph, b.I0));
+         }
+      } else if (first_step && merge && P.mesh_motion != 3) {
          DH_TRY(run_both(x, "wcell_plm_phi", kw, m.ntot, kpl, m.ntot));
       } else {
          if (first_step) {
@@ -734,7 +760,7 @@ struct Engine {
          }
          DH_TRY(run_ord(x, "plm_phi", kpl, m.ntot, b.ord[ORD_CELLS]));
       }
-      DH_TRY(topology<NQ>(true, reuse));
+      DH_TRY(topology<NQ>(true, reuse, rings));
       KFluxPhi<NQ, H> kp{m, P, dt, b.prim, b.gradp, b.gradr, b.gradz, b.piph, b.dphi, b.wiph,
                          b.dFp, b.emf_phi};
       KFluxTrans<NQ, H, 1> kt1{m, P, dt, b.F[0], b.prim, b.gradp, b.gradr, b.gradz, b.piph, b.dphi,
