@@ -1332,7 +1332,7 @@ struct RunOp {
       if (t < n) k(t);
    }
 };
-// A kernel over cells or faces by tiles.
+// A kernel that runs by tiles only.
 template <class K>
 struct TileOp {
    static constexpr int min_waves = 1;
@@ -1491,12 +1491,19 @@ struct GroupExec {
    {
       return n > 0 ? rec(RunOp<K>{k, n}) : DH_OK;
    }
+   // By elements whatever the members' annuli (a member's tiles are read
+   // through a pointer in device memory, which takes back what the scalar
+   // indices give, and short annuli leave lanes idle).  By elements against
+   // by tiles, ms a step: 16 planet disks of 96 and 128 rings 0.73 / 0.74 and
+   // 1.18 / 1.20, 8 of 512 rings 7.21 / 7.27; MHD disks 16 x (16 x 4)
+   // 0.94 / 0.97, 4 x (64 x 16) 4.97 / 4.99, 8 x (32 x 8) and 2 x (96 x 16)
+   // within 0.3% either way; 8 GRMHD disks of 32 x 8 3.21 / 3.27.
    template <class K>
    int run_tuned(const char *, const K &k, long n, const GroupOrder *, int, const int *)
    {
       if (n <= 0) return DH_OK;
-      if constexpr (ByElements<K>::value) return rec(RunOp<K>{k, n});
-      else return rec(TileOp<K>{k});
+      if constexpr (ByTilesOnly<K>::value) return rec(TileOp<K>{k});
+      else return rec(RunOp<K>{k, n});
    }
    int ring_start(const Mesh &m, const double *piph, int *I0)
    {

@@ -102,3 +102,53 @@ def test_ensemble_members_match_the_reference():
         ens.close()
         for r in runs:
             r.close()
+
+
+@pytest.mark.parametrize("graphs", [True, False])
+@pytest.mark.parametrize("cname,sizes", [
+    # copied ghost rings on both z sides, constrained transport with flips,
+    # edge means by 63-cell tiles; annuli from under one tile to a dozen
+    ("mhd_kep", [dict(Num_R=16, Num_Z=4), dict(Num_R=32, Num_Z=8),
+                 dict(Num_R=10, Num_Z=6, aspect=0.1)]),
+    ("gr_disk", [dict(Num_R=16, Num_Z=4, R_Min=8.0, R_Max=20.0, CFL=0.2, Riemann_Solver=2),
+                 dict(Num_R=24, Num_Z=6, R_Min=8.0, R_Max=20.0, CFL=0.2, Riemann_Solver=2)]),
+    # the smallest members: annuli of a few cells, polar axis
+    ("euler_yee", [dict(Num_R=24), dict(Num_R=6), dict(Num_R=13)]),
+])
+def test_ensembles_of_every_module_equal_their_own_runs(cname, sizes, graphs):
+    """The members' launches (by elements, grouped) against the same runs'
+    own launches (by elements or by tiles, some merged): the same kernel
+    bodies on the same data, bit for bit."""
+    from disco_amd.host_lib import Ensemble, HostRun
+    d = tempfile.mkdtemp(prefix="ensall_")
+    print(f"case ensemble {cname} {sizes}, graphs {graphs}", flush=True)
+
+    def open_all(tag):
+        return [HostRun(cname, state_io.write_par(
+            os.path.join(d, f"{tag}{i}"), configs.get(cname).par_dict(**s, Autotune=0)))
+            for i, s in enumerate(sizes)]
+    runs, solo = open_all("e"), open_all("s")
+    ens = Ensemble(runs, graphs=graphs)
+    try:
+        for n in range(6):
+            ens.step()
+            for i, r in enumerate(solo):
+                dt = r.getmindt()
+                assert dt == ens.dts[i], (n, i, dt, ens.dts[i])
+                r.timestep(dt)
+        ens.sync()
+        for i, (a, b) in enumerate(zip(runs, solo)):
+            pa, pb = os.path.join(d, f"a{i}.dstate"), os.path.join(d, f"b{i}.dstate")
+            a.write(pa)
+            b.write(pb)
+            x, y = state_io.read_state(pa), state_io.read_state(pb)
+            assert np.isfinite(x.prim).all()
+            for key in ("prim", "piph", "dphi", "wiph", "phi_flux"):
+                assert np.array_equal(getattr(x, key), getattr(y, key)), (
+                    i, key, np.abs(getattr(x, key) - getattr(y, key)).max())
+            print(f"  member {i}: annuli of {x.np_.min()} to {x.np_.max()} cells, identical",
+                  flush=True)
+    finally:
+        ens.close()
+        for r in runs + solo:
+            r.close()
