@@ -124,8 +124,7 @@ __device__ __forceinline__ void tile_wave(const K &k, const TileList &tl, int w,
 {
    if (w >= tl.n) return;
    Tile t = tl.t[w];
-   // (an ensemble's tile comes through a pointer in memory, whose load the
-   // compiler does not know to be uniform)
+   // (uniform over the wavefront)
    t.first = __builtin_amdgcn_readfirstlane(t.first);
    t.n = __builtin_amdgcn_readfirstlane(t.n);
    t.group = __builtin_amdgcn_readfirstlane(t.group);
@@ -137,6 +136,8 @@ __device__ __forceinline__ void tile_wave(const KEdgesCollectAvg &k, const TileL
 {
    if (w >= tl.n) return;
    Tile t = tl.t[w];
+   // (an ensemble's tile comes through a pointer in memory, whose load the
+   // compiler does not know to be uniform)
    t.first = __builtin_amdgcn_readfirstlane(t.first);
    t.n = __builtin_amdgcn_readfirstlane(t.n);
    const int a = __builtin_amdgcn_readfirstlane(t.group);
@@ -1396,8 +1397,8 @@ struct MindtOp {
    dh_params P;
    const double *prim, *piph, *dphi, *wiph;
    unsigned long long *out;
-   unsigned nb;
-   unsigned blocks() const { return nb; }
+   PaddedInt nb;
+   unsigned blocks() const { return (unsigned)nb; }
    __device__ __forceinline__ void run(unsigned b) const
    {
       mindt_block<NQ, H>(m, P, prim, piph, dphi, wiph, out, b, nb);
@@ -1493,11 +1494,11 @@ struct GroupExec {
    }
    // By elements whatever the members' annuli (a member's tiles are read
    // through a pointer in device memory, which takes back what the scalar
-   // indices give, and short annuli leave lanes idle).  By elements against
-   // by tiles, ms a step: 16 planet disks of 96 and 128 rings 0.73 / 0.74 and
-   // 1.18 / 1.20, 8 of 512 rings 7.21 / 7.27; MHD disks 16 x (16 x 4)
-   // 0.94 / 0.97, 4 x (64 x 16) 4.97 / 4.99, 8 x (32 x 8) and 2 x (96 x 16)
-   // within 0.3% either way; 8 GRMHD disks of 32 x 8 3.21 / 3.27.
+   // indices give, and short annuli leave lanes idle).  A step by elements
+   // against by tiles: 16 planet disks of 96 and 128 rings 1.5% shorter, 8 of
+   // 512 rings 0.8%; MHD disks 16 x (16 x 4) 3%, 4 x (64 x 16) 0.5%,
+   // 8 x (32 x 8) and 2 x (96 x 16) within 0.3% either way; 8 GRMHD disks of
+   // 32 x 8 2%.
    template <class K>
    int run_tuned(const char *, const K &k, long n, const GroupOrder *, int, const int *)
    {
@@ -1578,7 +1579,7 @@ template <int NQ, class H>
 static int ens_record_mindt(GroupExec *gx, Buffers *b, unsigned long long *out)
 {
    unsigned nb = nblocks(b->m.ntot) < 512 ? nblocks(b->m.ntot) : 512;
-   return gx->rec(MindtOp<NQ, H>{b->m, b->P, b->prim, b->piph, b->dphi, b->wiph, out, nb});
+   return gx->rec(MindtOp<NQ, H>{b->m, b->P, b->prim, b->piph, b->dphi, b->wiph, out, (int)nb});
 }
 
 template <int KIND>
@@ -1593,6 +1594,7 @@ struct dh_ens {
    int nm = 0;
    hipStream_t stream = nullptr;         // every member's work goes here while joined
    std::vector<EnsLaunch> plan;          // the timestep's launches
+   long tables = 0;                      // launch tables built so far
    bool graphs = false;
    hipGraphExec_t gexec = nullptr;
    StepArgs **d_dst = nullptr;           // each member's StepArgs
@@ -1635,8 +1637,13 @@ static void ens_release(dh_ens *e)
 // The ops of position i of every member's record as one launch (device
 // copies of the ops and the block table).
 // *changed tells whether the launch differs from what L held (then L is
-// rebuilt; otherwise its device copies stay as they are).
-static int ens_build_launch(const std::vector<GroupExec> &rec, size_t i, EnsLaunch &L,
+// rebuilt; otherwise its device copies stay as they are).  The ops are
+// compared byte by byte, so none of them has padding bytes (PaddedInt): with
+// them the minimum's table, and in MHD one of the step's, which took its
+// recorded graph with it, were freed, allocated and uploaded again in every
+// step (8 MHD disks of 32 x 8: 1.90 ms a step, now 1.78; 16 planet disks of
+// 32 rings 0.27, now 0.23).
+static int ens_build_launch(dh_ens *e, const std::vector<GroupExec> &rec, size_t i, EnsLaunch &L,
                             bool *changed)
 {
    int nm = (int)rec.size();
@@ -1650,6 +1657,7 @@ static int ens_build_launch(const std::vector<GroupExec> &rec, size_t i, EnsLaun
    }
    *changed = !(L.d_ops && L.tag == g0.tag && L.host == host && L.total == total);
    if (!*changed) return DH_OK;
+   ++e->tables;
    std::vector<int2> map;
    map.reserve(total);
    for (int m = 0; m < nm; ++m)
@@ -2005,6 +2013,10 @@ int dh_ens_create(dh_ctx *const *members, int n, dh_ens **out)
    return DH_OK;
 }
 
+// For the tests: how many launch tables the ensemble has built (an RK2 run
+// builds none after its first steps).
+long dhx_ens_tables(const dh_ens *e) { return e ? e->tables : -1; }
+
 int dh_ens_destroy(dh_ens *e)
 {
    ens_release(e);
@@ -2035,7 +2047,7 @@ int dh_ens_getmindt(dh_ens *e, double *dts)
       DH_TRY(DH_DISPATCH(b, ens_record_mindt, &rec[m], &b, e->d_min + m));
    }
    bool changed = false;
-   DH_TRY(ens_build_launch(rec, 0, e->mindt, &changed));
+   DH_TRY(ens_build_launch(e, rec, 0, e->mindt, &changed));
    k_fill_u64<<<(e->nm + 63) / 64, 64, 0, e->stream>>>(e->d_min, e->nm, 0x7FF0000000000000ULL);
    LAUNCH_CHECK();
    DH_TRY(ens_launch(e, e->mindt));
@@ -2075,7 +2087,7 @@ int dh_ens_timestep(dh_ens *e, const double *dts)
    e->plan.resize(nops);
    for (size_t i = 0; i < nops; ++i) {
       bool changed = false;
-      DH_TRY(ens_build_launch(rec, i, e->plan[i], &changed));
+      DH_TRY(ens_build_launch(e, rec, i, e->plan[i], &changed));
       if (changed) same = false;
    }
    if (!same) ens_drop_graph(e);
@@ -2148,7 +2160,7 @@ int dh_ens_add_diagnostics(dh_ens *e, int kind, const double *dts, const double 
       DH_TRY(rc);
    }
    bool changed = false;
-   DH_TRY(ens_build_launch(rec, 0, e->diag, &changed));
+   DH_TRY(ens_build_launch(e, rec, 0, e->diag, &changed));
    e->diag_kind = kind;
    HIPCHK(hipMemcpyAsync(e->d_diag, e->h_diag, sizeof(EnsDiagArgs) * e->nm, hipMemcpyHostToDevice,
                          e->stream));

@@ -519,7 +519,7 @@ struct KGrad {
    static constexpr int dim = DIM;
    static constexpr bool xcd_contiguous = DIM == 1;
    double PLM;
-   int num_c;
+   PaddedInt num_c;
    Faces F;
    const int *rng;
    const double *piph, *dphi, *prim, *gradp;
@@ -1009,7 +1009,7 @@ struct KUpdate {
    dh_params P;
    double RK;
    const double *dtp;
-   int first_step;
+   PaddedInt first_step;
    const PlanetSet *pls;
    const double *prim_in;
    double *prim;
@@ -1132,7 +1132,7 @@ struct KUpdate {
 // substep with (Ecarry), as the reference's cell arrays do.
 struct KEdgesCollect {
    Mesh m;
-   int ct;
+   PaddedInt ct;
    const double *dphi, *emf_phi;
    Faces Fr, Fz;
    const int *rngr, *rngz;
@@ -1318,7 +1318,7 @@ DHD void edges_post_face(const EdgeArgs &g, long c, int a, double *out)
 template <bool AVG>
 struct KEdgesFinal {
    EdgeArgs g;
-   int ct;
+   PaddedInt ct;
    const double *wiph, *emf_r, *emf_z;
    double *Eo, *Eown, *Ecarry;
    DHD TileList tiles() const { return g.m.tiles; }
@@ -1898,6 +1898,7 @@ DHD int bc_layers(const Mesh &m, int side)
 // The sides of one direction (r or z) whose ghost annuli are copied.
 struct BcSides {
    int n, side[2], diode[2], lines[2], layers[2];
+   int zero;  // (in place of padding bytes, PaddedInt)
    DHD unsigned rings() const
    {
       unsigned r = 0;

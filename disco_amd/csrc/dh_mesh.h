@@ -26,9 +26,20 @@ struct Tile {
    int group;      // annulus or annulus pair
    int dim;        // faces: 1 (r) or 2 (z); cells: 0
 };
+
+// An int that fills 8 bytes.  An ensemble compares the arguments of a launch
+// with those of the last step byte by byte, so its kernels hold no padding
+// bytes, whose values nothing determines.
+struct PaddedInt {
+   int v, zero;
+   PaddedInt() = default;
+   DHD PaddedInt(int n) : v(n), zero(0) {}
+   DHD operator int() const { return v; }
+};
+
 struct TileList {
    const Tile *t;
-   int n;
+   PaddedInt n;
 };
 
 struct Mesh {

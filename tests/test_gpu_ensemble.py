@@ -152,3 +152,36 @@ def test_ensembles_of_every_module_equal_their_own_runs(cname, sizes, graphs):
         ens.close()
         for r in runs + solo:
             r.close()
+
+
+@pytest.mark.parametrize("cname,over", [
+    ("euler_yee", {"Num_R": 24}), ("disk_planet", {"Num_R": 48}),
+    ("mhd_kep", {"Num_R": 12, "Num_Z": 4}),
+    ("gr_disk", {"Num_R": 12, "Num_Z": 4, "R_Min": 8.0, "R_Max": 20.0, "CFL": 0.2}),
+])
+def test_launch_tables_are_built_once(cname, over):
+    """The launches of an RK2 run have the same arguments in every step (dt,
+    planets and the minima lie in device memory), so their tables are built
+    in the first steps and stay: not one is freed, allocated and uploaded
+    again for bytes of an argument that hold no value."""
+    import ctypes as C
+    from disco_amd import capi
+    from disco_amd.host_lib import Ensemble, HostRun
+    d = tempfile.mkdtemp(prefix="enstab_")
+    print(f"case launch tables of {cname} {over}", flush=True)
+    tables = capi.lib().dhx_ens_tables
+    tables.argtypes, tables.restype = [C.c_void_p], C.c_long
+    runs = [HostRun(cname, state_io.write_par(
+        os.path.join(d, str(i)), configs.get(cname).par_dict(**over, Autotune=0))) for i in range(3)]
+    ens = Ensemble(runs)
+    try:
+        built = []
+        for _ in range(8):
+            ens.step()
+            built.append(tables(ens.ens))
+        print("  tables built by step:", built, flush=True)
+        assert built[2] > 0 and built[-1] == built[2], built
+    finally:
+        ens.close()
+        for r in runs:
+            r.close()
