@@ -1760,6 +1760,16 @@ int dh_destroy(dh_ctx *c)
    return DH_OK;
 }
 
+// For the tests: the cell count below which this context runs launches as
+// one (SMALL_MESH_CELLS), so that a small mesh can take a large one's sequence.
+int dhx_merge_below(dh_ctx *c, long cells)
+{
+   if (!c) return fail(DH_EINVAL, "null context");
+   c->x.drop_graph();
+   c->b.merge_below = cells;
+   return DH_OK;
+}
+
 int dh_create(const dh_grid *g, const dh_params *par, dh_ctx **out)
 {
    if (!g || !par || !out) return fail(DH_EINVAL, "null argument");

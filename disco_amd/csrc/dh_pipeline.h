@@ -64,14 +64,29 @@ struct OrderSet {
    int n = 0;
 };
 
-// Meshes below this many cells (ghosts included) run some independent
-// launches of a substep as one.
+// Meshes below this many cells (ghosts included) run launches of a substep
+// that share no data as one.  On small meshes every launch waits mostly on
+// its own latency (a dependent launch costs 5 us and more however little it
+// does); on large ones a launch fills the card by itself, and the merged
+// kernels' registers, those of the hungriest part, only cost waves: most of
+// all the relativistic fluxes' (three bodies of 256 registers in one).
+// A step merged against apart, ms:
+//   Euler   0.65M cells 0.513 / 0.531, 0.83M 0.580 / 0.601, 1.30M 0.892 / 0.928
+//   MHD     0.46M 1.14 / 1.24, 0.85M 2.02 / 2.10, 1.41M 3.29 / 3.34,
+//           2.2M 4.96 / 4.98, 3.1M 7.03 / 6.97
+//   GRMHD   0.41M (torus) 1.72 / 1.75, 0.54M 2.20 / 2.21, 0.62M 2.50 / 2.49,
+//           0.64M (disks) 2.33 / 2.34 and 2.48 / 2.47, 0.70M 2.86 / 2.79,
+//           0.76M 2.76 / 2.73, 0.88M 3.58 / 3.48, 1.03M 3.72 / 3.62
+// so the line lies at 5/8 of 2^20 cells for GRMHD.  The others' is anywhere
+// from 1.4M to 2.2M; it stays at 2^20, within 2% of the better side there.
 constexpr long SMALL_MESH_CELLS = 1L << 20;
+constexpr long SMALL_MESH_CELLS_GR = 5L << 17;
 
 struct Buffers {
    dh_params P;
    int nq = 0, nf = 0;
    bool mhd = false;
+   long merge_below = 0;  // SMALL_MESH_CELLS of the module
    Mesh m;
    int *Np = nullptr, *off = nullptr, *cjk = nullptr;
    double *r = nullptr, *z = nullptr;
@@ -412,6 +427,7 @@ int create_buffers(X &x, Buffers &b, const dh_grid *g, const dh_params &P)
    b.nq = P.num_c + P.num_n;
    b.mhd = P.hydro == DH_HYDRO_MHD || P.hydro == DH_HYDRO_GRMHD;
    b.nf = b.mhd ? 5 : 0;
+   b.merge_below = P.hydro == DH_HYDRO_GRMHD ? SMALL_MESH_CELLS_GR : SMALL_MESH_CELLS;
    int nq = b.nq;
    int nann = g->Nr * g->Nz;
    b.h_Np.assign(g->Np, g->Np + nann);
@@ -641,11 +657,8 @@ struct Engine {
       return DH_OK;
    }
 
-   // Whether launches that share no data go as one: on small meshes, where
-   // every launch waits mostly on its own latency (a dependent launch costs
-   // 5 us and more however little it does).  Above 2^20 cells a launch fills
-   // the card by itself and the merged kernels' registers only cost waves.
-   bool merged() const { return x.merges_launches() && b.m.ntot < SMALL_MESH_CELLS; }
+   // Whether launches that share no data go as one (SMALL_MESH_CELLS).
+   bool merged() const { return x.merges_launches() && b.m.ntot < b.merge_below; }
 
    // The same with the r and the z direction's launches as one.
    template <int NQ>
