@@ -1309,6 +1309,12 @@ static int do_faces(dh_ctx *c)
    Engine<HipExec> e{c->x, c->b};
    return e.template faces<NQ, H>();
 }
+template <int NQ, class H>
+static int do_flips(dh_ctx *c, double dt, double *Phi2, signed char *LR_r, signed char *LR_z)
+{
+   Engine<HipExec> e{c->x, c->b};
+   return e.template flips_only<NQ, H>(dt, Phi2, LR_r, LR_z);
+}
 
 // ---------------------------------------------------------------------------
 // Ensembles (dh_ens_*): independent meshes of one module selection, each
@@ -1758,6 +1764,13 @@ int dh_destroy(dh_ctx *c)
 {
    release(c);
    return DH_OK;
+}
+
+// For the tests: Engine::flips_only.
+int dhx_flips(dh_ctx *c, double dt, double *Phi2, signed char *LR_r, signed char *LR_z)
+{
+   if (!c || !Phi2 || !LR_r || !LR_z) return fail(DH_EINVAL, "null argument");
+   return DH_DISPATCH(c->b, do_flips, c, dt, Phi2, LR_r, LR_z);
 }
 
 // For the tests: the cell count below which this context runs launches as

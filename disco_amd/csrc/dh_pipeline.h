@@ -77,8 +77,8 @@ struct OrderSet {
 //   GRMHD   0.41M (torus) 1.72 / 1.75, 0.54M 2.20 / 2.21, 0.62M 2.50 / 2.49,
 //           0.64M (disks) 2.33 / 2.34 and 2.48 / 2.47, 0.70M 2.86 / 2.79,
 //           0.76M 2.76 / 2.73, 0.88M 3.58 / 3.48, 1.03M 3.72 / 3.62
-// so the line lies at 5/8 of 2^20 cells for GRMHD.  The others' is anywhere
-// from 1.4M to 2.2M; it stays at 2^20, within 2% of the better side there.
+// so the line lies at 5/8 of 2^20 cells for GRMHD.  The Newtonian modules'
+// is below where merging stops to gain (2 to 4% of a step at 1.1M to 1.4M).
 constexpr long SMALL_MESH_CELLS = 1L << 20;
 constexpr long SMALL_MESH_CELLS_GR = 5L << 17;
 
@@ -723,6 +723,31 @@ struct Engine {
       return DH_OK;
    }
 
+   // check_flipped and flip_fluxes (bfields.c:693-814) of every face track
+   // for faces moved by *dt: hand-overs of Phi and, alongside, of Phi2.
+   int flip_faces(const double *dt, double *Phi, double *Phi2)
+   {
+      const Mesh &m = b.m;
+      if constexpr (HasFlipTracks<X>::value) {
+         return x.flip_tracks(m, b.F[0], b.F[1], b.piph, b.wiph, dt, Phi, Phi2);
+      } else {
+         for (int dim = 1; dim <= 2; ++dim) {
+            int d = dim - 1;
+            if (!dim_active(m, dim)) continue;
+            if (dim == 1)
+               DH_TRY(run_ord(x, "flip_flags_r",
+                              KFlipFlags<1>{m, b.F[d], b.piph, b.wiph, dt, b.flag[d]},
+                              b.F[d].n, b.ord[ORD_FACES_R]));
+            else
+               DH_TRY(run_ord(x, "flip_flags_z",
+                              KFlipFlags<2>{m, b.F[d], b.piph, b.wiph, dt, b.flag[d]},
+                              b.F[d].n, b.ord[ORD_FACES_Z]));
+            DH_TRY(x.flips(m, dim, b.F[d], b.flag[d], Phi, Phi2));
+         }
+         return DH_OK;
+      }
+   }
+
    // The conserved state and the magnetic fluxes of a substep: in, the RK
    // blend's other state, and out (the buffer that holds the substep's
    // result, which the kernels after the update read); pflip is the copy of
@@ -846,24 +871,7 @@ struct Engine {
       }
       if (!both || !mhd) DH_TRY(run_ord(x, "update", ku, m.ntot, b.ord[ORD_CELLS]));
       if constexpr (mhd) {
-         if constexpr (HasFlipTracks<X>::value) {
-            if (first_step)
-               DH_TRY(x.flip_tracks(m, b.F[0], b.F[1], b.piph, b.wiph, dt, st.pout, st.pflip));
-         } else if (first_step) {
-            for (int dim = 1; dim <= 2; ++dim) {
-               int d = dim - 1;
-               if (!dim_active(m, dim)) continue;
-               if (dim == 1)
-                  DH_TRY(run_ord(x, "flip_flags_r",
-                                 KFlipFlags<1>{m, b.F[d], b.piph, b.wiph, dt, b.flag[d]},
-                                 b.F[d].n, b.ord[ORD_FACES_R]));
-               else
-                  DH_TRY(run_ord(x, "flip_flags_z",
-                                 KFlipFlags<2>{m, b.F[d], b.piph, b.wiph, dt, b.flag[d]},
-                                 b.F[d].n, b.ord[ORD_FACES_Z]));
-               DH_TRY(x.flips(m, dim, b.F[d], b.flag[d], st.pout, st.pflip));
-            }
-         }
+         if (first_step) DH_TRY(flip_faces(dt, st.pout, st.pflip));
          // with the learned guess cons2prim waits for the model's guesses,
          // which need the cells' conserved field first
          bool learned = IsGR<H>::value && P.c2p_guess != DH_C2P_GUESS_PREVIOUS;
@@ -966,6 +974,27 @@ struct Engine {
       if (d0 <= 0.0) d0 = 1.0e100;
       if (v < d0) d0 = v;
       *dt = d0 * b.P.cfl;
+      return DH_OK;
+   }
+
+   // For the tests: the flips of faces moved by dt, on the context's Phi and
+   // on Phi2 (host, [5][ntot], in and out); the orientations after them.
+   template <int NQ, class H>
+   int flips_only(double dt, double *Phi2, signed char *LR_r, signed char *LR_z)
+   {
+      if (!b.mhd) return fail(DH_EINVAL, "face flips need the MHD fields");
+      size_t bytes = sizeof(double) * 5 * (size_t)b.m.ntot;
+      StepArgs sa;
+      memset(&sa, 0, sizeof sa);
+      sa.dt[0] = dt;
+      DH_TRY((faces<NQ, H>()));
+      DH_TRY(x.set_step(b.step, sa));
+      DH_TRY(x.put(b.rkPhi, Phi2, bytes));
+      DH_TRY(flip_faces(b.step->dt, b.Phi, b.rkPhi));
+      DH_TRY(x.get(Phi2, b.rkPhi, bytes));
+      if (b.F[0].n) DH_TRY(x.get(LR_r, b.F[0].LR, (size_t)b.F[0].n));
+      if (b.F[1].n) DH_TRY(x.get(LR_z, b.F[1].LR, (size_t)b.F[1].n));
+      b.topo_valid = false;
       return DH_OK;
    }
 

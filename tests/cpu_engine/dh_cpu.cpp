@@ -235,6 +235,13 @@ static int do_faces(dh_ctx *c)
 }
 
 template <int NQ, class H>
+static int do_flips(dh_ctx *c, double dt, double *Phi2, signed char *LR_r, signed char *LR_z)
+{
+   Engine<HostExec> e{c->x, c->b};
+   return e.template flips_only<NQ, H>(dt, Phi2, LR_r, LR_z);
+}
+
+template <int NQ, class H>
 static int do_grads(dh_ctx *c, int dim, double *out)
 {
    Engine<HostExec> e{c->x, c->b};
@@ -297,6 +304,11 @@ extern "C" long dhx_check_orders(dh_ctx *c)
    return checked;
 }
 
+extern "C" int dhx_flips(dh_ctx *c, double dt, double *Phi2, signed char *LR_r, signed char *LR_z)
+{
+   if (!c || !Phi2 || !LR_r || !LR_z) return fail(DH_EINVAL, "null argument");
+   return DH_DISPATCH(c->b, do_flips, c, dt, Phi2, LR_r, LR_z);
+}
 extern "C" long dhx_flip_count(dh_ctx *c) { return c ? c->x.flipped : -1; }
 extern "C" long dhx_bc_rings(dh_ctx *c) { return c ? c->x.bc_rings : -1; }
 extern "C" long dhx_bc_misses(dh_ctx *c) { return c ? c->x.bc_misses : -1; }

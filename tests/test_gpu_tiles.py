@@ -61,8 +61,8 @@ def test_long_annuli_step_as_the_host_build(cname, over):
 @pytest.mark.parametrize("aspect", [0.5, 0.12, 0.06, 0.03])
 def test_flips_of_strong_shear(aspect):
     """Keplerian shear of about a cell a step flips most faces: tracks of
-    fewer faces than a flip batch (256), about as many, and several batches,
-    with runs that cross batches and the track's closure.  Steps from common
+    fewer faces than a flip batch (256) and of several batches, in whole
+    steps (the lengths around a batch: test_gpu_flips).  Steps from common
     states: a trajectory of this mesh is ill-conditioned (the host build's
     own moves by 1e-10 under a one-ulp change of libm)."""
     import sys
