@@ -848,8 +848,12 @@ struct TimerRow {
 // Launch variants of a kernel that runs over cells or faces (run_tuned):
 // 0 storage order with the workgroups dealt to the XCDs round-robin (the
 // hardware's order), 1 storage order with each XCD given a contiguous
-// eighth (block_of), and for a kernel that runs by tiles 2 + s the group order s of the kernel's OrderSet
-// (strips of annuli, XCD-contiguous).  All give the same results.
+// eighth (block_of), and for a kernel that runs by tiles 2 + s the order s of
+// its OrderSet (strips of annuli, XCD-contiguous).  All give the same results.
+// By elements (the fluxes, meshes of short annuli) the strip orders gained
+// nothing: with them and without, ms a step, Kerr torus 128 x 64 6.24 / 6.24,
+// GRMHD disk 112 x 28 10.38 / 10.40, MHD disks 127 x 31 6.95 / 6.96 and
+// 192 x 48 22.72 / 22.70.
 struct TuneRow {
    std::string name;
    int nvar = 0, chosen = -1, dflt = 0;
@@ -936,9 +940,11 @@ struct HipExec {
       return t;
    }
 
+   static bool takes_tiles(const TileList &tl, long n) { return by_tiles(tl, n); }
+
    // A kernel over cells or faces in one of its launch variants (TuneRow).
    template <class K>
-   int run_tuned(const char *name, const K &k, long n, const GroupOrder *ords, int nord,
+   int run_tuned(const char *name, const K &k, long n, const TileList *ords, int nord,
                  const int *strips)
    {
       if (n <= 0) return DH_OK;
@@ -965,7 +971,7 @@ struct HipExec {
          Bracket b(*this, name);
          if constexpr (!ByElements<K>::value)
             if (tiled) {
-               TileList tl = v < 2 ? tiles_of(k) : ords[v - 2].tiles;
+               TileList tl = v < 2 ? tiles_of(k) : ords[v - 2];
                long nt = (long)tl.n * 64;
                k_tiles<K><<<v == 0 ? nblocks(nt) : nblocks_xcd(nt), TPB, 0, stream>>>(k, tl, v != 0);
             }
@@ -1506,7 +1512,7 @@ struct GroupExec {
    // 8 x (32 x 8) and 2 x (96 x 16) within 0.3% either way; 8 GRMHD disks of
    // 32 x 8 2%.
    template <class K>
-   int run_tuned(const char *, const K &k, long n, const GroupOrder *, int, const int *)
+   int run_tuned(const char *, const K &k, long n, const TileList *, int, const int *)
    {
       if (n <= 0) return DH_OK;
       if constexpr (ByTilesOnly<K>::value) return rec(TileOp<K>{k});

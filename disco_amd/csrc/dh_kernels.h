@@ -67,41 +67,13 @@ struct IsGR<GRMHD<NQ>> {
    static constexpr bool value = true;
 };
 
-// Traversal orders of a kernel's elements.  The elements come in groups
-// that are contiguous in storage (the cells of an annulus, the faces of an
-// annulus pair), and an order visits whole groups in some sequence: thread
-// t does element elem(t).  Every element's work is independent of when it
-// runs (owner-computes, no atomics), so an order changes only which
-// elements share an L2 at a time, never a result.
-//   first[p]  storage index of the first element of the p-th visited group
-//   pos[p]    thread index at which that group starts (pos[ng] = n)
-//   chunk[c]  the p whose range holds thread ORDER_CHUNK * c, so that a
-//             thread finds its group after a step or two from there
-constexpr int ORDER_CHUNK = 256;
-struct GroupOrder {
-   const int *first, *pos, *chunk;
-   int ng;
-   TileList tiles;  // the same sequence in tiles (what a wavefront-per-tile launch takes)
-   DHD long elem(long t) const
-   {
-      int p = chunk[t / ORDER_CHUNK];
-      while (pos[p + 1] <= t) ++p;
-      return first[p] + (t - pos[p]);
-   }
-};
-
 // Kernels over cells or faces take an element and its group (and, for both
 // face lists as one range, its direction): at(e, g, dim).  A launch by tiles
-// (one wavefront per tile of tiles()) hands them the tile's group; the
-// element alone, operator()(e), looks its group up.
-
-// A kernel run in a group order, element by element.
-template <class K>
-struct Grouped {
-   K k;
-   GroupOrder o;
-   DHD void operator()(long t) const { k(o.elem(t)); }
-};
+// (one wavefront per tile, of tiles() or of another list of the same elements
+// in another order) hands them the tile's group; the element alone,
+// operator()(e), looks its group up.  Every element's work is independent of
+// when it runs (owner-computes, no atomics), so an order changes only which
+// elements share an L2 at a time, never a result.
 
 // Two kernels that share no data in one launch: threads [0, n1) run the
 // first over its elements, the rest the second over its own.

@@ -6,6 +6,9 @@
 // test suite instantiates a host executor to run the same bodies on the CPU
 // against the oracle.  X provides
 //   run(name, kernel, n)          kernel(t) for t in [0, n)
+//   run_tuned(name, kernel, n, orders, count, strips)   the same in any order, or by the
+//                                 tiles of kernel.tiles() or of one of the orders
+//   takes_tiles(tiles, n)         whether n elements in these tiles run by tiles
 //   ring_start(m, piph, I0)       start cell of every annulus
 //   flip_tracks(m, Fr, Fz, piph, wiph, dtp, Phi, rkPhi)   flags and hand-overs of
 //                                 every track's flipped faces; or
@@ -55,11 +58,12 @@ inline int fail(int code, const char *fmt, ...)
 // order the z neighbours of a gather are far apart in time and in the
 // strip orders both neighbours are close; the strip height trades the
 // annuli between the two.  With one layer every strip order is the storage
-// order, and a set has none.
+// order, and a set has none; nor has it where the executor does not run the
+// kind by tiles (takes_tiles).
 enum { ORD_CELLS = 0, ORD_FACES_R = 1, ORD_FACES_Z = 2, ORD_EDGES = 3, ORD_KINDS = 4 };
 constexpr int MAX_ORDERS = 4;
 struct OrderSet {
-   GroupOrder o[MAX_ORDERS];
+   TileList o[MAX_ORDERS];
    int strip[MAX_ORDERS];
    int n = 0;
 };
@@ -268,38 +272,9 @@ int put_tiles(X &x, TileList &out, const GroupSeq &s, int most = TILE)
    return DH_OK;
 }
 
-// One group order on the device from the host lists of the visited groups'
-// storage starts and sizes.
-template <class X>
-int put_order(X &x, GroupOrder &o, const GroupSeq &seq)
-{
-   const std::vector<int> &first = seq.first, &size = seq.size;
-   int ng = (int)first.size();
-   std::vector<int> pos(ng + 1, 0);
-   for (int p = 0; p < ng; ++p) pos[p + 1] = pos[p] + size[p];
-   long n = pos[ng];
-   std::vector<int> chunk((size_t)(n / ORDER_CHUNK + 1), 0);
-   for (int p = 0, c = 0; c < (int)chunk.size(); ++c) {
-      long t = (long)c * ORDER_CHUNK;
-      while (p < ng - 1 && pos[p + 1] <= t) ++p;
-      chunk[c] = p;
-   }
-   int *d[3] = {nullptr, nullptr, nullptr};
-   DH_TRY(alloc_n(x, &d[0], sizeof(int) * (size_t)(ng > 0 ? ng : 1)));
-   DH_TRY(alloc_n(x, &d[1], sizeof(int) * (size_t)(ng + 1)));
-   DH_TRY(alloc_n(x, &d[2], sizeof(int) * chunk.size()));
-   if (ng > 0) DH_TRY(x.put(d[0], first.data(), sizeof(int) * (size_t)ng));
-   DH_TRY(x.put(d[1], pos.data(), sizeof(int) * (size_t)(ng + 1)));
-   DH_TRY(x.put(d[2], chunk.data(), sizeof(int) * chunk.size()));
-   o.first = d[0];
-   o.pos = d[1];
-   o.chunk = d[2];
-   o.ng = ng;
-   return put_tiles(x, o.tiles, seq);
-}
-
-// The storage-order tiles of the cells and faces and the strip orders of every kind (OrderSet).  fI holds the host copies of
-// both face lists' pair offsets.
+// The storage-order tiles of the cells and faces and the strip orders of
+// every kind (OrderSet).  fI holds the host copies of both face lists' pair
+// offsets.
 template <class X>
 int build_orders(X &x, Buffers &b, const std::vector<int> *fI)
 {
@@ -338,6 +313,8 @@ int build_orders(X &x, Buffers &b, const std::vector<int> *fI)
       }
       if (b.mhd) DH_TRY(put_tiles(x, m.etiles, edges));
    }
+   const TileList *storage[ORD_KINDS] = {&m.tiles, &b.F[0].tiles, &b.F[1].tiles, &m.etiles};
+   const long n[ORD_KINDS] = {m.ntot, b.F[0].n, b.F[1].n, b.mhd ? (long)b.F[0].n + b.F[1].n : 0};
    for (int S : strip_heights(Nz)) {
       // (j, k) of the cells' groups in this strip order
       std::vector<std::pair<int, int>> order;
@@ -348,8 +325,9 @@ int build_orders(X &x, Buffers &b, const std::vector<int> *fI)
       sequences(order, seq);
       for (int kind = 0; kind < ORD_KINDS; ++kind) {
          OrderSet &os = b.ord[kind];
+         if (n[kind] == 0 || !x.takes_tiles(*storage[kind], n[kind])) continue;
          if (os.n >= MAX_ORDERS) return fail(DH_EINVAL, "too many traversal orders");
-         DH_TRY(put_order(x, os.o[os.n], seq[kind]));
+         DH_TRY(put_tiles(x, os.o[os.n], seq[kind]));
          os.strip[os.n] = S;
          ++os.n;
       }

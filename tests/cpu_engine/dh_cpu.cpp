@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <utility>
 #include <vector>
 
 #include "disco_hip.h"
@@ -30,20 +31,39 @@ struct HostExec {
       for (long t = 0; t < n; ++t) k(t);
       return DH_OK;
    }
-   // A kernel with launch variants (the GPU tuner's numbering: 0 and 1 the
-   // storage order, 2 + s group order s).  DH_CPU_ORDER = v runs every such
-   // kernel in variant v where the kernel has it (strip orders visit every
-   // element once, in another sequence: the results must not change).
+   // A kernel by a list of tiles, each element with its tile's group.
    template <class K>
-   int run_tuned(const char *, const K &k, long n, const GroupOrder *ords, int nord, const int *)
+   static int walk(const K &k, const TileList &tl)
+   {
+      for (int w = 0; w < tl.n; ++w)
+         for (int i = 0; i < tl.t[w].n; ++i) k.at(tl.t[w].first + i, tl.t[w].group, tl.t[w].dim);
+      return DH_OK;
+   }
+   template <class K1, class K2>
+   static int walk_storage(const KBoth<K1, K2> &k)
+   {
+      DH_TRY(walk_storage(k.k1));
+      return walk_storage(k.k2);
+   }
+   template <class K>
+   static int walk_storage(const K &k) { return walk(k, k.tiles()); }
+   static bool takes_tiles(const TileList &, long) { return true; }
+   template <class K1, class K2>
+   static int walk_order(const KBoth<K1, K2> &k, const TileList &) { return walk_storage(k); }
+   template <class K>
+   static int walk_order(const K &k, const TileList &tl) { return walk(k, tl); }
+   // A kernel with launch variants (the GPU tuner's numbering: 0 and 1 the
+   // storage order, 2 + s order s).  DH_CPU_ORDER = v runs every such kernel
+   // in variant v where the kernel has it: 0 by elements, 1 by the tiles of
+   // the storage order, 2 + s by those of order s (every order visits each
+   // element once: the results must not change).
+   template <class K>
+   int run_tuned(const char *, const K &k, long n, const TileList *ords, int nord, const int *)
    {
       const char *e = getenv("DH_CPU_ORDER");
       int v = e ? atoi(e) : 0;
-      if (v >= 2 && v - 2 < nord) {
-         Grouped<K> g{k, ords[v - 2]};
-         for (long t = 0; t < n; ++t) g(t);
-         return DH_OK;
-      }
+      if (v >= 2 && v - 2 < nord) return walk_order(k, ords[v - 2]);
+      if (v == 1) return walk_storage(k);
       for (long t = 0; t < n; ++t) k(t);
       return DH_OK;
    }
@@ -279,26 +299,52 @@ int dhx_riemann(dh_ctx *c, const double *pL, const double *pR, double r, const d
 }
 
 
-// Every group order of every kind visits each element of its range exactly
-// once: returns the number of orders checked, or -1 at the first that does
-// not.
+// Whether a list of tiles (at most `most` elements each) visits every one of
+// n elements exactly once and hands each its group and direction.
+template <class G>
+static bool tiles_cover(const TileList &tl, long n, int most, const G &group_of)
+{
+   std::vector<char> seen((size_t)n, 0);
+   long total = 0;
+   for (int w = 0; w < tl.n; ++w) {
+      const Tile &t = tl.t[w];
+      if (t.n < 1 || t.n > most || t.first < 0 || (long)t.first + t.n > n) return false;
+      for (long e = t.first; e < (long)t.first + t.n; ++e) {
+         if (seen[(size_t)e] || group_of(e) != std::make_pair(t.group, t.dim)) return false;
+         seen[(size_t)e] = 1;
+         ++total;
+      }
+   }
+   return total == n;
+}
+
+// The tiles of every kind, in storage order and in every strip order, cover
+// their elements: returns the number of strip orders checked, or -1.
 extern "C" long dhx_check_orders(dh_ctx *c)
 {
    if (!c) return -1;
    Buffers &b = c->b;
-   long nkind[ORD_KINDS] = {b.m.ntot, b.F[0].n, b.F[1].n, (long)b.F[0].n + b.F[1].n};
+   const long nr = b.F[0].n, nz = b.F[1].n;
+   auto cells = [&](long e) { return std::make_pair(b.m.cjk[e], 0); };
+   auto rfaces = [&](long e) { return std::make_pair(b.F[0].pf[e], 1); };
+   auto zfaces = [&](long e) { return std::make_pair(b.F[1].pf[e], 2); };
+   auto edges = [&](long e) { return e < nr ? rfaces(e) : zfaces(e - nr); };
+   auto covers = [&](int kind, const TileList &tl) {
+      return kind == ORD_CELLS      ? tiles_cover(tl, b.m.ntot, TILE, cells)
+             : kind == ORD_FACES_R  ? tiles_cover(tl, nr, TILE, rfaces)
+             : kind == ORD_FACES_Z  ? tiles_cover(tl, nz, TILE, zfaces)
+                                    : tiles_cover(tl, nr + nz, TILE, edges);
+   };
+   if (!covers(ORD_CELLS, b.m.tiles) || (nr && !covers(ORD_FACES_R, b.F[0].tiles)) ||
+       (nz && !covers(ORD_FACES_Z, b.F[1].tiles)))
+      return -1;
+   if (b.mhd && (!covers(ORD_EDGES, b.m.etiles) ||
+                 !tiles_cover(b.m.atiles, b.m.ntot, TILE - 1, cells)))
+      return -1;
    long checked = 0;
    for (int kind = 0; kind < ORD_KINDS; ++kind)
       for (int s = 0; s < b.ord[kind].n; ++s) {
-         const GroupOrder &o = b.ord[kind].o[s];
-         long n = nkind[kind];
-         if (o.pos[o.ng] != n) return -1;
-         std::vector<char> seen((size_t)n, 0);
-         for (long t = 0; t < n; ++t) {
-            long e = o.elem(t);
-            if (e < 0 || e >= n || seen[(size_t)e]) return -1;
-            seen[(size_t)e] = 1;
-         }
+         if (!covers(kind, b.ord[kind].o[s])) return -1;
          ++checked;
       }
    return checked;

@@ -43,6 +43,22 @@ def load_golden(name):
 GOLDEN_CASES = list(make_golden.CASES)
 
 
+def host_initial(cname, over):
+    """(config, in.par dict, initial state) by this project's own driver on
+    the host build of the engine (no reference build, no GPU)."""
+    import subprocess
+    import tempfile
+    from disco_amd import state_io
+    sys.path.insert(0, os.path.join(HERE, "cpu_engine"))
+    import build as cpu_build
+    cfg = configs.get(cname)
+    par = cfg.par_dict(**over)
+    d = tempfile.mkdtemp(prefix="init_")
+    state_io.write_par(d, par)
+    subprocess.run([cpu_build.build_driver(cname), "0"], cwd=d, check=True, capture_output=True)
+    return cfg, par, state_io.read_state(os.path.join(d, "output.dstate"))
+
+
 def rel_l1(x: np.ndarray, y: np.ndarray) -> float:
     """Relative L1 difference sum|x-y| / sum|y| (0 when both are 0)."""
     den = np.abs(y).sum()
