@@ -111,20 +111,37 @@ def b_alg(nq: int, nf: int) -> int:
     return 40 * (nq + nf + 1)
 
 
+# The launches of small meshes that run several kernels as one.
+MERGED = {
+    "wcell_plm_phi": ("wcell", "plm_phi"),
+    "wcell_plm_phi_rings": ("wcell", "plm_phi", "ring_start"),
+    "plm_phi_rings": ("plm_phi", "ring_start"),
+    "faces": ("faces_r", "faces_z"),
+    "grad": ("grad_r", "grad_z"),
+    "flux_phi_r": ("flux_phi", "flux_r"),
+    "flux": ("flux_phi", "flux_r", "flux_z"),
+    "update_edges_collect": ("update", "edges_collect"),
+    "edges_final_line_steps": ("edges_final", "line_steps_r", "line_steps_z"),
+    "update_B_edge_segments": ("update_B", "edge_segments"),
+}
+
+
 def kernel_bytes(name: str, nq: int, mhd: bool, nt: int, nr: int, nfr: int, nfz: int,
-                 zlayer: int = 0) -> float:
+                 zlayer: int = 0, zcopied: int = 4, gr: bool = False) -> float:
     """Algorithmic bytes of one launch of a kernel: every array element the
     kernel needs read once and every output element written once (8-byte
     doubles, 4-byte indices, 1-byte face orientations).  nt counts all cells
     (ghosts included), nr the real ones, nfr/nfz the r and z faces; zlayer is
-    the cell count of one z ghost layer (0 when no z side is copied).
+    the cell count of one z ghost layer (0 when no z side is copied), zcopied
+    the copied z layers of both sides; gr tells GRMHD, whose edge EMFs are
+    stored before their means over two cells are taken.
 
     Per face the topology holds L, R (int), LR (byte) and up, dA, phic, dphi
     (double); every cell has two merge steps per direction (int) and its
     annulus index cjk (int)."""
-    merged = {"wcell_plm_phi": ("wcell", "plm_phi"), "flux_phi_r": ("flux_phi", "flux_r")}
-    if name in merged:                  # two launches run as one on small meshes
-        return sum(kernel_bytes(k, nq, mhd, nt, nr, nfr, nfz, zlayer) for k in merged[name])
+    if name in MERGED:                  # launches run as one on small meshes
+        return sum(kernel_bytes(k, nq, mhd, nt, nr, nfr, nfz, zlayer, zcopied, gr)
+                   for k in MERGED[name])
     d, i = 8, 4
     nql = nq - 3 if mhd else nq         # components the fluxes update
     nf = {"r": nfr, "z": nfz}.get(name[-1:], 0)
@@ -139,6 +156,8 @@ def kernel_bytes(name: str, nq: int, mhd: bool, nt: int, nr: int, nfr: int, nfz:
     if name in ("ranges_r", "ranges_z"):
         return d * nt + i * nt + steps
     if name in ("faces_r", "faces_z"):
+        # the merge steps in (on small meshes out: they are formed here), the
+        # positions and extents in, the faces out
         return steps + i * nt + d * 2 * nt + nf * (2 * i + 1 + 4 * d)
     if name in ("grad_r", "grad_z"):
         return steps + i * nt + nf * (2 * i + 2 * d) + d * nt * (2 + 3 * nq)
@@ -147,12 +166,14 @@ def kernel_bytes(name: str, nq: int, mhd: bool, nt: int, nr: int, nfr: int, nfz:
     if name in ("flux_r", "flux_z"):
         return (nf * (2 * i + 2 * d) + d * nt * (2 + 3 * nq) + d * nql * nf
                 + (3 * d * nf if mhd else 0))
+    epre = 16 if gr else 8              # edge numbers a cell between the two edge kernels
     if name == "edges_collect":
-        return d * 21 * nt + 2 * steps + i * nt + 3 * d * nfa
+        # emf_phi (4) and dphi in, Epre out per cell, the face EMFs in
+        return d * (epre + 5) * nt + 2 * steps + i * nt + 3 * d * nfa
     if name == "edges_final":
-        # Epre (16), wiph, piph and dphi in, Eo and Eown (4 + 4) out per cell;
+        # Epre, wiph, piph and dphi in, Eo and Eown (4 + 4) out per cell;
         # per owned face its cells and orientation and its E_phi in
-        return d * 27 * nt + 2 * steps + i * nt + nfa * (d + 2 * i + 1)
+        return d * (epre + 11) * nt + 2 * steps + i * nt + nfa * (d + 2 * i + 1)
     if name == "update_B":
         # Phi in and out, rkPhi on the second substep only (mean 2.5 per cell)
         return d * (12.5 + 4) * nt + 2 * steps + i * nt + nfa * (2 * i + 1)
@@ -179,20 +200,18 @@ def kernel_bytes(name: str, nq: int, mhd: bool, nt: int, nr: int, nfr: int, nfz:
     if name == "bfaces_c2p":
         return (2 * steps + i * nt + d * 10 * nt + nfa * (2 * i + 1 + d)
                 + d * nq * nr * 2)
-    if name in ("flip_flags_r", "flip_flags_z"):
-        return nf * (2 * i + 2) + 2 * d * nt
     if name == "flips":
-        return nfa
+        # the faces' cells and orientations and their owners' positions and
+        # velocities in (hand-overs, as many as the shear makes, not counted)
+        return nfa * (2 * i + 1) + 2 * d * nt
     if name == "mindt":
         return d * (nq * nr + 3 * nt) + i * nt
     if name == "diagnostics":          # prim (rho..B), piph, dphi in; Qrz out
         return d * (8 + 2) * nt + i * nt
-    if name == "bc_scan":               # one z side: positions of both layers' rings
-        return 2 * zlayer * (4 * d + i)
-    if name == "bc_fill":               # one z ghost layer from the layer inside it
-        return zlayer * (d * (2 * nq + 4) + i)
-    if name == "copy":                  # cons -> rkcons (and Phi -> rkPhi): mean launch
-        return 2 * d * nt * (nq + 5) / 2 if mhd else 2 * d * nt * nq
+    if name == "bc_scan":               # both z sides: positions of each layer's rings
+        return zcopied * zlayer * (4 * d + i)
+    if name == "bc_fill":               # every z ghost layer from the layer inside it
+        return zcopied * zlayer * (d * (2 * nq + 4) + i)
     return 0.0
 
 
@@ -653,6 +672,7 @@ def main(argv=None):
     z_copied = any(bc[s] in (configs.BC_ZEROGRAD, configs.BC_DIODE) for s in (2, 3))
     r_copied = any(bc[s] in (configs.BC_ZEROGRAD, configs.BC_DIODE) for s in (0, 1))
     zlayer = ntot // nz_tot if z_copied and not r_copied else 0
+    zcopied = sum(ng for s in (2, 3) if bc[s] in (configs.BC_ZEROGRAD, configs.BC_DIODE))
 
     roofline = None
     kernels = None
@@ -672,7 +692,7 @@ def main(argv=None):
         kernels = {}
         for k in range(n.value):
             nm = bytes(names[k]).split(b"\0")[0].decode()
-            alg = kernel_bytes(nm, nq, mhd, ntot, ncell, nfr, nfz, zlayer)
+            alg = kernel_bytes(nm, nq, mhd, ntot, ncell, nfr, nfz, zlayer, zcopied, gr)
             mean_s = ms[k] / max(calls[k], 1) * 1e-3
             kernels[nm] = {"ms_per_step": ms[k] / tsteps, "launches_per_step": calls[k] / tsteps,
                            "mean_launch_ms": mean_s * 1e3,
