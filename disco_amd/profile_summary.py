@@ -21,9 +21,20 @@ import sqlite3
 import sys
 from collections import defaultdict
 
-# kernel symbol (as rocprofv3 prints it) -> the engine's timer name
+# kernel symbol (as rocprofv3 prints it) -> the engine's timer name, first
+# match; the launches of small meshes that run several kernels as one first
 _NAMES = [
-    (r"KBoth<dh::KWcell<", "wcell_plm_phi"), (r"KBoth<dh::KFluxPhi<", "flux_phi_r"),
+    (r"k_run<dh::K(BfacesC2p|Wcell)<", "init"),
+    (r"k_elems_rings<dh::KBoth<dh::KWcell<", "wcell_plm_phi_rings"),
+    (r"k_elems_rings<dh::KPlmPhi<", "plm_phi_rings"),
+    (r"KBoth<dh::KWcell<", "wcell_plm_phi"),
+    (r"KBoth<dh::KRangesFaces<1>", "faces"), (r"KRangesFaces<1>", "faces_r"),
+    (r"KBoth<dh::KGrad<", "grad"),
+    (r"KBoth<dh::KFluxPhi<[^()]*KBoth<dh::KFluxTrans<", "flux"),
+    (r"KBoth<dh::KFluxPhi<", "flux_phi_r"),
+    (r"KBoth<dh::KUpdate<", "update_edges_collect"),
+    (r"KBoth<dh::KEdgesFinal<", "edges_final_line_steps"),
+    (r"KBoth<dh::KUpdateB,", "update_B_edge_segments"),
     (r"KPlmPhi<", "plm_phi"),
     (r"k_ring_start", "ring_start"),
     (r"KCellRanges<1>", "ranges_r"), (r"KCellRanges<2>", "ranges_z"),
@@ -32,24 +43,24 @@ _NAMES = [
     (r"KFluxPhi<", "flux_phi"),
     (r"KFluxTrans<.*, 1>", "flux_r"), (r"KFluxTrans<.*, 2>", "flux_z"),
     (r"KEdgesCollect", "edges_collect"),
-    (r"KEdgesFinal", "edges_final"),
+    (r"KEdgesFinal<", "edges_final"),
     (r"KUpdateB", "update_B"),
     (r"KLineSteps<1>", "line_steps_r"), (r"KLineSteps<2>", "line_steps_z"),
     (r"KEdgeSegments", "edge_segments"), (r"KEdgeAdjust", "edge_adjust"),
     (r"KUpdate<", "update"),
-    (r"KFlipFlags<1>", "flip_flags_r"), (r"KFlipFlags<2>", "flip_flags_z"),
     (r"k_flips", "flips"),
     (r"KBfacesC2p<", "bfaces_c2p"),
-    (r"KBcScan", "bc_scan"), (r"KBcFill<", "bc_fill"),
-    (r"k_mindt<", "mindt"), (r"k_bc_scan", "bc_scan"), (r"k_diag<", "diagnostics"),
-    (r"KDiagAvg", "diag_avg"),
+    (r"k_bc_rings", "bc_scan"), (r"k_bc_columns<", "bc_fill"),
+    (r"k_c2p_guess<", "c2p_guess"), (r"KC2p<", "c2p"),
+    (r"k_mindt<", "mindt"), (r"k_diag<", "diagnostics"), (r"k_report", "report"),
+    (r"KDiagAvg", "diag_avg"), (r"k_set_step\b", "set_step"),
     (r"KWcell<", "wcell"), (r"KWcellAvg", "wcell"),
     (r"KInitCells<", "init"),
 ]
 
 
 def timer_name(kernel: str) -> str:
-    head = kernel.split("(")[0] if kernel.startswith("k_") else kernel
+    head = re.sub(r"^void ", "", kernel).split("(")[0]
     for pat, name in _NAMES:
         if re.search(pat, head):
             return name
@@ -65,53 +76,56 @@ def _rows(db: str, sql: str):
 
 
 def functor_of(kernel: str) -> str:
-    """The functor a k_run / k_run_xcd launch runs, whatever its launch
-    variant (storage order, XCD-contiguous, or wrapped in a group order);
-    other kernels are their own."""
-    m = re.match(r"void k_run(?:_xcd)?<(.*)>\((.*), long\)$", kernel)
-    if not m:
-        return kernel
-    f = m.group(2)
-    g = re.match(r"dh::Grouped<(.*)>$", f)
-    return g.group(1).strip() if g else f.strip()
+    """The functor a launch by elements or by tiles runs (k_run, k_elems,
+    k_tiles, k_elems_rings), whose launch variants differ only in the order of
+    the work; other kernels are their own."""
+    m = re.match(r"void k_(?:run|elems|tiles|elems_rings)<(.*)>\((?:.*)\)$", kernel)
+    return _template_args(m.group(1)).strip() if m else kernel
 
 
-def after_tuning(rows):
-    """The rows (kernel, dispatch_id, value) of each functor's last launch
-    variant from the dispatch after the last one of any other variant of the
-    same functor: the launches that follow the launch tuner's sweep."""
-    last = defaultdict(lambda: -1)
-    for name, did, _ in rows:
-        last[name] = max(last[name], did)
-    by_functor = defaultdict(list)
-    for name in last:
-        by_functor[functor_of(name)].append(name)
-    keep = {}
-    for names in by_functor.values():
-        final = max(names, key=lambda n: last[n])
-        keep[final] = max([last[n] for n in names if n != final], default=-1)
-    return [r for r in rows if r[0] in keep and r[1] > keep[r[0]]]
+def _template_args(s: str) -> str:
+    """The part of `s` before its outermost closing '>' when the argument
+    list's own templates follow it."""
+    depth = 0
+    for i, ch in enumerate(s):
+        depth += ch == "<"
+        depth -= ch == ">"
+        if depth < 0:
+            return s[:i]
+    return s
 
 
-def kernel_stats(db: str, tuned: bool = False):
+def after_tuning(rows, tune_steps):
+    """The rows (kernel, dispatch_id, value) that follow the launch tuner's
+    sweep over the run's first tune_steps timesteps.  A kernel's launch
+    variants share one symbol, so the sweep is told apart by its timesteps:
+    each begins with one k_set_step, and the first untuned one with the
+    (tune_steps + 1)-th."""
+    starts = sorted(did for name, did, _ in rows if re.match(r"(?:void )?k_set_step\b", name))
+    if len(starts) <= tune_steps:
+        raise ValueError(f"the run has {len(starts)} timesteps, its sweep {tune_steps}")
+    return [r for r in rows if r[1] >= starts[tune_steps]]
+
+
+def kernel_stats(db: str, tune_steps: int = 0):
     """{kernel: (calls, total_ns, mean_ns)} of a --kernel-trace database
-    (tuned: only the launches after the tuner's sweep)."""
+    (tune_steps: only the launches after the tuner's sweep over so many steps)."""
     rows = _rows(db, "select name, dispatch_id, duration from kernels")
-    if tuned:
-        rows = after_tuning(rows)
+    if tune_steps:
+        rows = after_tuning(rows, tune_steps)
     acc = defaultdict(list)
     for name, _, dur in rows:
         acc[name].append(dur)
     return {k: (len(v), sum(v), sum(v) / len(v)) for k, v in acc.items()}
 
 
-def counter_means(db: str, counter: str, tuned: bool = False):
-    """{kernel: (dispatches, mean value)} of one --pmc counter (tuned: only
-    the launches after the tuner's sweep)."""
+def counter_means(db: str, counter: str, tune_steps: int = 0):
+    """{kernel: (dispatches, mean value)} of one --pmc counter (tune_steps:
+    only the launches after the tuner's sweep over so many steps)."""
     rows = _rows(db, "select kernel_name, dispatch_id, value from counters_collection "
                      f"where counter_name = '{counter}'")
-    if tuned:
-        rows = after_tuning(rows)
+    if tune_steps:
+        rows = after_tuning(rows, tune_steps)
     acc = defaultdict(list)
     for name, _, value in rows:
         acc[name].append(value)
@@ -133,10 +147,12 @@ def cmd_kernels(args):
     lines = [f"# Kernel trace: {args.title}", ""]
     if args.cmd:
         lines += ["Command:", "", "```", args.cmd, "```", ""]
-    lines += ["## After the launch tuner's sweep", "",
-              "Each kernel in the launch variant the tuner kept, from its first launch after "
-              "the last launch of any other variant (the warmup and timed steps).", ""]
-    lines += _kernel_table(kernel_stats(args.db, tuned=True))
+    if args.tune_steps:
+        lines += ["## After the launch tuner's sweep", "",
+                  f"The launches after the first {args.tune_steps} timesteps, each kernel in the "
+                  "variant the tuner kept (the warmup and timed steps, and the steps under the "
+                  "event timers).", ""]
+        lines += _kernel_table(kernel_stats(args.db, args.tune_steps))
     lines += ["", "## Every dispatch of the run", ""]
     lines += _kernel_table(kernel_stats(args.db))
     with open(args.out, "w") as f:
@@ -157,8 +173,8 @@ def _copy_factor(fetch_db: str, write_db: str):
 
 def cmd_traffic(args):
     rf, wf, probe = _copy_factor(args.copy_fetch, args.copy_write)
-    fetch = counter_means(args.fetch, "FETCH_SIZE", tuned=args.tuned)
-    write = counter_means(args.write, "WRITE_SIZE", tuned=args.tuned)
+    fetch = counter_means(args.fetch, "FETCH_SIZE", args.tune_steps)
+    write = counter_means(args.write, "WRITE_SIZE", args.tune_steps)
     kernels = {}
     for name in sorted(set(fetch) | set(write)):
         tn = timer_name(name)
@@ -178,7 +194,7 @@ def cmd_traffic(args):
     out = {"workload": args.workload,
            "counters": "FETCH_SIZE and WRITE_SIZE (KiB per dispatch), one rocprofv3 --pmc run each",
            "launches": ("each kernel in the launch variant the tuner kept, after its sweep"
-                        if args.tuned else "every dispatch"),
+                        if args.tune_steps else "every dispatch"),
            "scale": {"read": rf, "write": wf,
                      "probe": f"1 GiB device-to-device copy ({probe.split('(')[0]})"},
            "command": args.cmd, "kernels": kernels}
@@ -207,8 +223,8 @@ def cmd_fp64(args):
     (one --pmc run with FP64_COUNTERS) times 64 lanes, an FMA counting two
     operations, over the kernel's mean duration in a --kernel-trace run of
     the same workload (the launches after the tuner's sweep, in the variant
-    it kept; every launch variant of a kernel runs the same instructions)."""
-    stats = kernel_stats(args.trace, tuned=True)
+    it kept; the variants of a kernel run the same instructions)."""
+    stats = kernel_stats(args.trace, args.tune_steps)
     # instruction counts per functor: every launch variant runs the same code
     per = {}
     for c in FP64_COUNTERS:
@@ -256,14 +272,15 @@ def main(argv=None):
     for a in ("--fetch", "--write", "--copy-fetch", "--copy-write", "--workload", "--out"):
         t.add_argument(a, required=True)
     t.add_argument("--cmd", default="")
-    t.add_argument("--tuned", action="store_true",
-                   help="only the launches after the launch tuner's sweep")
     sub.add_parser("copy-probe")
     f = sub.add_parser("fp64")
     for a in ("--pmc", "--trace", "--out"):
         f.add_argument(a, required=True)
     f.add_argument("--title", default="")
     f.add_argument("--cmd", default="")
+    for q in (k, t, f):
+        q.add_argument("--tune-steps", type=int, default=0,
+                       help="the run's launch-tuning steps, whose launches are left out")
     args = ap.parse_args(argv)
     {"kernels": cmd_kernels, "traffic": cmd_traffic, "copy-probe": cmd_copy_probe,
      "fp64": cmd_fp64}[args.what](args)
