@@ -93,7 +93,11 @@ struct ByElements<KBoth<K1, K2>> {
    static constexpr bool value = ByElements<K1>::value || ByElements<K2>::value;
 };
 // Whether a kernel runs by tiles always (its lanes take values from each
-// other).
+// other).  A merged launch with such a part runs by tiles as a whole, the
+// conserved update beside the edges' collection for one, also on short
+// annuli: with the update by elements there a step of the MHD disks of
+// 32 x 8 to 80 x 20 rings took as long (0.356 / 0.358, 0.598 / 0.596,
+// 1.140 / 1.144, 2.024 / 2.027 ms).
 template <class K, class = void>
 struct ByTilesOnly {
    static constexpr bool value = false;
@@ -695,7 +699,9 @@ __global__ __launch_bounds__(MINDT_TPB) void k_mindt(Mesh m, dh_params P, const 
    if (threadIdx.x == 0) {
       // (no fence: both are device-scope atomics and this one is issued after
       // the other has returned; a fence writes the whole L2 back, 55 us a
-      // call over the 2048 workgroups of a large mesh)
+      // call when 2048 workgroups each had one.  The order of the two relaxed
+      // atomics is this hardware's, which completes a returning device-scope
+      // atomic where every XCD sees it, not the memory model's.)
       if (atomicAdd(&st->done, 1u) == gridDim.x - 1) {
          unsigned long long v = atomicExch(&st->min, MINDT_NONE);
          atomicExch(&st->done, 0u);
@@ -1518,6 +1524,11 @@ struct GroupExec {
       if constexpr (ByTilesOnly<K>::value) return rec(TileOp<K>{k});
       else return rec(RunOp<K>{k, n});
    }
+   template <class K1, class K2>
+   int run_tuned(const char *, const KBoth<K1, K2> &, long, const TileList *, int, const int *)
+   {
+      return fail(DH_EINVAL, "an ensemble keeps launches apart");
+   }
    int ring_start(const Mesh &m, const double *piph, int *I0)
    {
       return rec(RingStartOp{m, piph, I0});
@@ -1979,7 +1990,6 @@ int dh_c2p_grad_noalloc(const float *params, const float *X, const float *Y, lon
                   C2P_NOALLOC_ROWS, n);
    float *s = nullptr;
    DH_TRY(scratch_of_current_device(&s));
-   hipStream_t st = (hipStream_t)stream;
    return HipExec::mlp_launch(MlpBatch{params, X, Y, nullptr, (int)n, nullptr, nullptr}, s, grad,
                               MlpAdam{}, loss, nullptr, (hipStream_t)stream);
 }

@@ -93,7 +93,8 @@ DHD double polar_adjust(double phip, double phim, double Pmax)
 // low parts: within 0.51 ulp of the exact power, where the device's pow is
 // within 1 ulp, at about 15 instead of 150 instructions (pow was half of
 // the cell update's arithmetic in the disks: four calls per planet and two
-// per energy frame).  Zero, infinities and NaN give what pow gives.
+// per energy frame).  Zero, +infinity and NaN give what pow gives, and so do
+// negative numbers, but -infinity gives NaN where pow gives +infinity.
 DHD double pow_3_2(double r)
 {
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -1394,32 +1394,33 @@ int c2p_grad(X &x, const float *prm, const float *Xh, const float *Yh, long n, f
       DH_TRY(x.get(grad_out, g, sizeof(float) * C2PNET_NPARAM));
       if (loss_out) DH_TRY(x.get(loss_out, loss, sizeof(float)));
       return DH_OK;
+   } else {
+      DH_TRY(alloc_n(x, &idx, sizeof(int) * n));
+      DH_TRY(alloc_n(x, &act, sizeof(float) * C2PNET_ROW * n));
+      DH_TRY(alloc_n(x, &loss, sizeof(float) * n));
+      DH_TRY(alloc_n(x, &g, sizeof(float) * C2PNET_NTRAIN));
+      std::vector<int> hidx(n);
+      for (long i = 0; i < n; ++i) hidx[i] = (int)i;
+      DH_TRY(x.put(dX, Xh, sizeof(float) * C2PNET_IN * n));
+      DH_TRY(x.put(dY, Yh, sizeof(float) * C2PNET_OUT * n));
+      DH_TRY(x.put(dp, prm, sizeof(float) * C2PNET_NPARAM));
+      DH_TRY(x.put(idx, hidx.data(), sizeof(int) * n));
+      MlpBatch B{dp, dX, dY, idx, (int)n, act, loss};
+      DH_TRY(x.run("c2p_row", KMlpRow{B}, n));
+      DH_TRY(x.run("c2p_grad", KMlpGrad{B, g}, C2PNET_NTRAIN));
+      std::vector<float> hg(C2PNET_NTRAIN), hl(n);
+      DH_TRY(x.get(hg.data(), g, sizeof(float) * C2PNET_NTRAIN));
+      DH_TRY(x.get(hl.data(), loss, sizeof(float) * n));
+      for (int q = 0; q < C2PNET_NPARAM; ++q)
+         grad_out[q] = (q >= C2PNET_TRAIN0 && q < C2PNET_TRAIN0 + C2PNET_NTRAIN)
+                           ? hg[q - C2PNET_TRAIN0] : 0.0f;
+      if (loss_out) {
+         double s = 0.0;
+         for (long i = 0; i < n; ++i) s += hl[i];
+         *loss_out = (float)(s / (2.0 * n));
+      }
+      return DH_OK;
    }
-   DH_TRY(alloc_n(x, &idx, sizeof(int) * n));
-   DH_TRY(alloc_n(x, &act, sizeof(float) * C2PNET_ROW * n));
-   DH_TRY(alloc_n(x, &loss, sizeof(float) * n));
-   DH_TRY(alloc_n(x, &g, sizeof(float) * C2PNET_NTRAIN));
-   std::vector<int> hidx(n);
-   for (long i = 0; i < n; ++i) hidx[i] = (int)i;
-   DH_TRY(x.put(dX, Xh, sizeof(float) * C2PNET_IN * n));
-   DH_TRY(x.put(dY, Yh, sizeof(float) * C2PNET_OUT * n));
-   DH_TRY(x.put(dp, prm, sizeof(float) * C2PNET_NPARAM));
-   DH_TRY(x.put(idx, hidx.data(), sizeof(int) * n));
-   MlpBatch B{dp, dX, dY, idx, (int)n, act, loss};
-   DH_TRY(x.run("c2p_row", KMlpRow{B}, n));
-   DH_TRY(x.run("c2p_grad", KMlpGrad{B, g}, C2PNET_NTRAIN));
-   std::vector<float> hg(C2PNET_NTRAIN), hl(n);
-   DH_TRY(x.get(hg.data(), g, sizeof(float) * C2PNET_NTRAIN));
-   DH_TRY(x.get(hl.data(), loss, sizeof(float) * n));
-   for (int q = 0; q < C2PNET_NPARAM; ++q)
-      grad_out[q] = (q >= C2PNET_TRAIN0 && q < C2PNET_TRAIN0 + C2PNET_NTRAIN)
-                        ? hg[q - C2PNET_TRAIN0] : 0.0f;
-   if (loss_out) {
-      double s = 0.0;
-      for (long i = 0; i < n; ++i) s += hl[i];
-      *loss_out = (float)(s / (2.0 * n));
-   }
-   return DH_OK;
 }
 
 // Trains the learned guess on (X, Y) (host arrays, n rows): normalisation

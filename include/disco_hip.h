@@ -317,7 +317,9 @@ int dh_enable_graphs(dh_ctx *ctx, int on);
  *                     member: planets[m * DH_MAX_PLANETS * DH_PLANET_STRIDE
  *                     ...] are member m's npl planets after the step;
  *   dh_ens_destroy    gives every member its own stream back.
- * The members' results equal what dh_timestep gives each of them alone. */
+ * The members' results equal what dh_timestep gives each of them alone, bit
+ * for bit (in the Kerr metric on a small mesh, whose merged launches round a
+ * few operations otherwise when it is stepped alone, to rounding). */
 typedef struct dh_ens dh_ens;
 int dh_ens_create(dh_ctx *const *members, int n, dh_ens **out);
 int dh_ens_destroy(dh_ens *ens);
@@ -332,10 +334,11 @@ int dh_ens_sync(dh_ens *ens);
  * order on one core).  Every kernel of the step that runs over cells or
  * faces can be launched in several traversal orders: storage order with the
  * workgroups dealt to the XCDs round-robin (variant 0) or in contiguous
- * eighths (1), or whole annuli (annulus pairs) taken in strips of S layers
- * of z, the strips one after another, r after r within a strip and z
- * fastest (2, 3, ...; S = 4, 8, 16 or all layers).  Results are the same
- * in every order.  dh_autotune makes the next `steps` timesteps (eager,
+ * eighths (1), or, for the kernels that run by tiles of 64 elements of one
+ * annulus (annuli of about 500 cells and more; not the fluxes), whole annuli
+ * (annulus pairs) taken in strips of S layers of z, the strips one after
+ * another, r after r within a strip and z fastest (2, 3, ...; S = 4, 8, 16 or
+ * all layers).  Results are the same in every order.  dh_autotune makes the next `steps` timesteps (eager,
  * never recorded) tuning steps: in tuning step s every such kernel runs
  * all its launches of the step in variant s mod (its variant count), timed
  * with events, so that each variant is timed over whole steps; then each
