@@ -330,22 +330,22 @@ int dh_ens_add_diagnostics(dh_ens *ens, int kind, const double *dts, const doubl
 int dh_ens_enable_graphs(dh_ens *ens, int on);
 int dh_ens_sync(dh_ens *ens);
 
-/* Launch tuner (no counterpart in the reference, whose loops run in one
- * order on one core).  Every kernel of the step that runs over cells or
- * faces can be launched in several traversal orders: storage order with the
- * workgroups dealt to the XCDs round-robin (variant 0) or in contiguous
- * eighths (1), or, for the kernels that run by tiles of 64 elements of one
- * annulus (annuli of about 500 cells and more; not the fluxes), whole annuli
- * (annulus pairs) taken in strips of S layers of z, the strips one after
- * another, r after r within a strip and z fastest (2, 3, ...; S = 4, 8, 16 or
- * all layers).  Results are the same in every order.  dh_autotune makes the next `steps` timesteps (eager,
- * never recorded) tuning steps: in tuning step s every such kernel runs
- * all its launches of the step in variant s mod (its variant count), timed
- * with events, so that each variant is timed over whole steps; then each
- * kernel keeps its fastest (steps at least the largest variant count time
- * them all; steps = 0 keeps the choices made so far).  Until a kernel is
- * tuned it runs in variant 0, or 1 for the kernels that gather from the
- * next annulus in r.
+/* Launch tuner (no counterpart in the reference, whose loops run in one order
+ * on one core).  Every kernel of the step that runs over cells or faces can
+ * be launched in several traversal orders: storage order with the workgroups
+ * dealt to the XCDs round-robin (variant 0) or in contiguous eighths (1), or,
+ * for the kernels that run by tiles of 64 elements of one annulus (annuli of
+ * about 500 cells and more; not the fluxes), whole annuli (annulus pairs)
+ * taken in strips of S layers of z, the strips one after another, r after r
+ * within a strip and z fastest (2, 3, ...; S = 4, 8, 16 or all layers).
+ * Results are the same in every order.  dh_autotune makes the next `steps`
+ * timesteps (eager, never recorded) tuning steps: in tuning step s every such
+ * kernel runs all its launches of the step in variant s mod (its variant
+ * count), timed with events, so that each variant is timed over whole steps;
+ * then each kernel keeps its fastest (steps at least the largest variant
+ * count time them all; steps = 0 keeps the choices made so far).  Until a
+ * kernel is tuned it runs in variant 0, or 1 for the kernels that gather from
+ * the next annulus in r.
  * dh_read_tuning reports up to `cap` kernels: the chosen variant, its
  * strip height (0 for variants 0 and 1), and the mean launch time of the
  * chosen and of the untuned variant over the tuning steps (-1 if none).
