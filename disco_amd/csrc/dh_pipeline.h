@@ -73,7 +73,8 @@ struct OrderSet {
 // its own latency (a dependent launch costs 5 us and more however little it
 // does); on large ones a launch fills the card by itself, and the merged
 // kernels' registers, those of the hungriest part, only cost waves: most of
-// all the relativistic fluxes' (three bodies of 256 registers in one).
+// all the relativistic fluxes' (three bodies of 256 registers in one, which
+// spills 320 where each alone spills 72 to 100).
 // A step merged against apart, ms:
 //   Euler   0.65M cells 0.513 / 0.531, 0.83M 0.580 / 0.601, 1.30M 0.892 / 0.928
 //   MHD     0.46M 1.14 / 1.24, 0.85M 2.02 / 2.10, 1.41M 3.29 / 3.34,
